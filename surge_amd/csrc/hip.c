@@ -903,22 +903,15 @@ sg_err sg_gpu_run_rmsnorm_gated_chunk(sg_gpu *g, void *y, void *z, void *out, vo
                                             g->stream), outs, 1);
 }
 
+/* RoPE inverse frequencies theta^(-2i/rd), in double (reference
+ * metal.m:4027-4037, ref.c:561-602). */
+static void rope_inv_freq(double inv[SGK_ROPE_HALF], uint32_t rd, float theta) {
+    for (uint32_t i = 0; i < rd / 2; i++) inv[i] = pow((double)theta, -2.0 * (double)i / (double)rd);
+}
+
 /* Causal chunk attention (surge.h:787-788): query token t (position base+t)
  * over cache positions 0..base+t, through the split-K kernels with the
  * prefill split policy. */
-/* RoPE cos | sin per position for positions 0 .. npos-1, rd = rope_dim
- * floats each: angle and trig in double, stored f32 (reference
- * metal.m:4027-4037, ref.c:561-602). */
-static void rope_table(float *t, uint32_t npos, uint32_t rd, float theta) {
-    const uint32_t half = rd / 2;
-    for (uint32_t p = 0; p < npos; p++)
-        for (uint32_t i = 0; i < half; i++) {
-            const double ang = (double)p * pow((double)theta, -2.0 * (double)i / (double)rd);
-            t[(uint64_t)p * rd + i] = (float)cos(ang);
-            t[(uint64_t)p * rd + half + i] = (float)sin(ang);
-        }
-}
-
 sg_err sg_gpu_run_attn_prefill(sg_gpu *g, void *q, void *k, void *v, void *out, const uint32_t p[8]) {
     if (!g || !q || !k || !v || !out || !p) return (sg_err){"gpu: attn_prefill got a NULL argument"};
     uint32_t pp[8] = {p[0], p[1], p[2], 0, p[5], 0, 1, 0};
@@ -989,37 +982,28 @@ sg_err sg_gpu_run_attn_chunk(sg_gpu *g, void *in, void *w, void *kv, void *out, 
         return (sg_err){"gpu: attn_chunk: buffers must not overlap"};
     void *ins[3] = {in, w, kv}, *outs[2] = {kv, out};
     if (sg_failed(e = push(ins, 3))) return e;
-    /* scratch: step descriptors, the RoPE table for positions 0 .. cap-1, a
-     * working copy of the rows (the prep normalises q in place) and the key
-     * splits' partials */
-    const uint64_t steps_b = ((uint64_t)n * sizeof(sgk_step) + 255) / 256 * 256, cs_b = (cap * rd * 4 + 255) / 256 * 256;
-    const uint64_t work_b = n * row * 4, ah = (uint64_t)n * nh * SGK_PREFILL_SPLITS;
+    /* scratch: step descriptors, the chunk's RoPE rows, the normed and roped q
+     * (the caller's rows stay as they are) and the key splits' partials */
+    const uint64_t steps_b = ((uint64_t)n * sizeof(sgk_step) + 255) / 256 * 256, cs_b = ((uint64_t)n * rd * 4 + 255) / 256 * 256;
+    const uint64_t q_f = (uint64_t)n * nh * hd, ah = (uint64_t)n * nh * SGK_PREFILL_SPLITS;
     void *t;
-    if (sg_failed(e = scratch(g, steps_b + cs_b + work_b + ah * (2 + hd) * 4, &t))) return e;
-    sgk_step *hs = calloc(n, sizeof *hs);
-    float *ht = malloc(cap * rd * 4);
-    hipError_t he = hs && ht ? hipSuccess : hipErrorOutOfMemory;
-    if (he == hipSuccess) {
-        for (uint32_t z = 0; z < n; z++) hs[z].pos = base + z;
-        rope_table(ht, (uint32_t)cap, rd, fbits(p[6]));
-        he = hipMemcpy(t, hs, (uint64_t)n * sizeof *hs, hipMemcpyHostToDevice);
-        if (he == hipSuccess) he = hipMemcpy((char *)t + steps_b, ht, cap * rd * 4, hipMemcpyHostToDevice);
-    }
-    free(hs);
-    free(ht);
-    HIPCHK(he, "attn_chunk descriptors and RoPE table");
+    if (sg_failed(e = scratch(g, steps_b + cs_b + (q_f + ah * (2 + hd)) * 4, &t))) return e;
     hipStream_t s = g->stream;
     float *cs = (float *)((char *)t + steps_b), *work = (float *)((char *)t + steps_b + cs_b);
-    float *mm = work + n * row, *ss = mm + ah, *aa = ss + ah;
-    HIPCHK(hipMemcpyAsync(work, DEV(in), work_b, hipMemcpyDeviceToDevice, s), "attn_chunk rows");
-    const float *wn = DEV(w);
+    float *aa = work + q_f, *mm = aa + ah * hd, *ss = mm + ah;
+    const float *wn = DEV(w), *rows = DEV(in);
     uint16_t *kc = DEV(kv);
+    double inv[SGK_ROPE_HALF];
+    rope_inv_freq(inv, rd, fbits(p[6]));
     sgk_attn A = {0};
     A.q = work; A.kc = kc; A.vc = kc + kvh; A.m = mm; A.s = ss; A.acc = aa; A.out = DEV(out);
-    A.gate = work + hd; A.steps = t; A.n_heads = nh; A.n_kv = nkv; A.hd = hd; A.rope_dim = rd;
-    A.q_stride = 2 * hd; A.q_tok = (uint32_t)row; A.out_tok = nh * hd; A.max_splits = SGK_PREFILL_SPLITS;
+    A.src = rows; A.src_tok = (uint32_t)row; A.src_stride = 2 * hd;
+    A.gate = rows + hd; A.gate_tok = (uint32_t)row; A.gate_stride = 2 * hd;
+    A.steps = t; A.n_heads = nh; A.n_kv = nkv; A.hd = hd; A.rope_dim = rd;
+    A.q_stride = hd; A.q_tok = nh * hd; A.out_tok = nh * hd; A.max_splits = SGK_PREFILL_SPLITS;
     A.ntok = n; A.seq = (uint32_t)cap; A.scale = (float)(1.0 / sqrt((double)hd)); A.prefill = 1;
-    he = sgk_attn_prep(&A, wn, wn + hd, cs, fbits(p[7]), s);
+    hipError_t he = sgk_rope_rows(inv, rd, base, n, cs, t, s);
+    if (he == hipSuccess) he = sgk_attn_prep(&A, wn, wn + hd, cs, base, fbits(p[7]), s);
     if (he == hipSuccess) he = sgk_attn_flash(&A, s);
     return finish(g, he, outs, 2);
 }
@@ -1469,15 +1453,14 @@ sg_err sg_gpu_state_new(sg_gpu *g, const sg_model *m, uint32_t max_ctx) {
      * (reference metal.m:4027-4037, ref.c:561-602). */
     uint32_t rd = c->rope_dim ? c->rope_dim : 2;
     if (!sg_failed(e)) e = dalloc(g, (uint64_t)max_ctx * rd * 4, (void **)&g->cs_table);
-    if (!sg_failed(e)) {
-        float *t = malloc((uint64_t)max_ctx * rd * 4);
-        if (!t) e = (sg_err){"gpu: out of host memory"};
-        else {
-            rope_table(t, max_ctx, rd, c->rope_theta);
-            if (hipMemcpy(g->cs_table, t, (uint64_t)max_ctx * rd * 4, hipMemcpyHostToDevice) != hipSuccess)
-                e = (sg_err){"gpu: RoPE table upload failed"};
-            free(t);
-        }
+    /* (check_model holds an attention model's rope_dim to an even number up to
+     * head_dim; without attention layers nothing reads the table) */
+    if (!sg_failed(e) && rd % 2 == 0 && rd / 2 <= SGK_ROPE_HALF) {
+        double inv[SGK_ROPE_HALF];
+        rope_inv_freq(inv, rd, c->rope_theta);
+        hipError_t he = sgk_rope_rows(inv, rd, 0, max_ctx, g->cs_table, NULL, g->stream);
+        if (he == hipSuccess) he = hipStreamSynchronize(g->stream);
+        if (he != hipSuccess) e = errf("gpu: RoPE table: %s", hipGetErrorString(he));
     }
     if (!sg_failed(e) && hipHostMalloc((void **)&g->h_step, sizeof(sgk_step), 0) != hipSuccess) e = (sg_err){"gpu: hipHostMalloc failed"};
     if (!sg_failed(e) && hipHostMalloc((void **)&g->h_logits, (uint64_t)c->vocab * 4, 0) != hipSuccess) e = (sg_err){"gpu: hipHostMalloc failed"};
@@ -1828,7 +1811,7 @@ static hipError_t prefill_chunk(sg_gpu *g, uint32_t base, uint32_t n) {
             A.seq = base + n;       /* keys of the chunk's last token: the flash pass splits deep chunks */
             A.scale = (float)(1.0 / sqrt((double)hd)); A.prefill = 1;
             A.kv_ps = hd; A.kv_hs = (uint64_t)g->max_ctx * hd;
-            if ((e = sgk_attn_prep(&A, L->qn, L->kn, g->cs_table, c->rms_eps, s)) != hipSuccess) return e;
+            if ((e = sgk_attn_prep(&A, L->qn, L->kn, g->cs_table, 0, c->rms_eps, s)) != hipSuccess) return e;
             if (hd == 64 || hd == 128 || hd == 256) {
                 if ((e = sgk_attn_flash(&A, s)) != hipSuccess) return e;
             } else {

@@ -128,7 +128,14 @@ typedef struct {
     uint16_t *kc, *vc;          /* f16 caches (layout: kv_ps, kv_hs below) */
     float *m, *s, *acc;         /* partials */
     float *out;                 /* combine output [ntok][n_heads*hd] */
-    const float *gate;          /* combine: q rows again (gate half), or NULL */
+    const float *gate;          /* combine: the output gate's rows, or NULL */
+    uint32_t gate_tok, gate_stride; /* its strides per token and head (0: as q) */
+    /* prep: where the projection's rows (q|gate|k|v) are read when not in place:
+     * token z's at src + z*src_tok, query head h's at + h*src_stride, k and v
+     * after the last head's; q is then written to a->q (NULL: q holds the rows
+     * and is normalised in place) */
+    const float *src;
+    uint32_t src_tok, src_stride;
     const sgk_step *steps;
     uint32_t n_heads, n_kv, hd, rope_dim, q_stride, q_tok, out_tok;
     uint32_t seq, n_splits, max_splits, ntok;
@@ -155,9 +162,16 @@ typedef struct {
 } sgk_attn;
 
 /* q_norm/k_norm + RoPE on each head, K and V stored f16 at each token's
- * position. cs_table is [max_ctx][rope_dim] (cos | sin per position). */
+ * position. cs_table holds cos | sin rows [rope_dim] from position cs0 on. */
 hipError_t sgk_attn_prep(const sgk_attn *a, const float *qn, const float *kn,
-                         const float *cs_table, float eps, hipStream_t s);
+                         const float *cs_table, uint32_t cs0, float eps, hipStream_t s);
+/* RoPE cos | sin rows of positions base .. base+n-1 (cs [n][rope_dim]): angle
+ * and trig in double, stored f32, from the inverse frequencies inv[rope_dim/2]
+ * (host memory, read before return; rope_dim <= 2 * SGK_ROPE_HALF); and, with
+ * steps, the rows' step descriptors {0, base + z}. */
+#define SGK_ROPE_HALF 128u
+hipError_t sgk_rope_rows(const double *inv, uint32_t rope_dim, uint32_t base, uint32_t n, float *cs,
+                         sgk_step *steps, hipStream_t s);
 /* Split-K GQA partials: workgroup (split, kv head, token) serves all
  * n_heads/n_kv query heads of the group (grid x = max_splits with steps).
  * With fuse_prep the prep above is done inside (q in LDS; the split holding

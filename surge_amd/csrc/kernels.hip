@@ -1157,21 +1157,52 @@ __device__ __forceinline__ size_t kv_at(const sgk_attn &a, uint32_t pos, uint32_
 static inline sgk_attn kv_resolved(const sgk_attn *a) {
     sgk_attn b = *a;
     if (!b.kv_ps) { b.kv_ps = b.n_kv * b.hd; b.kv_hs = b.hd; }
+    if (!b.gate_stride) { b.gate_tok = b.q_tok; b.gate_stride = b.q_stride; }
     return b;
+}
+
+// RoPE rows: one thread per (position, frequency). Bound by the latency of one
+// double sincos; the host loop it replaces took 0.78 us per position (32
+// frequencies, one core: 25 ms of a 26.7 ms attention chunk at 32k keys). The
+// inverse frequencies come from the host so that the angle, and with it the
+// stored float, is the same one the host's table had.
+struct rope_inv { double f[SGK_ROPE_HALF]; };
+__global__ void __launch_bounds__(TPB) k_rope_rows(rope_inv inv, uint32_t half, uint32_t base, uint32_t n, float *cs,
+                                                   sgk_step *steps) {
+    const uint64_t i = (uint64_t)blockIdx.x * TPB + threadIdx.x;
+    const uint32_t z = (uint32_t)(i / half), f = (uint32_t)(i % half);
+    if (z >= n) return;
+    double s, c;
+    sincos((double)(base + z) * inv.f[f], &s, &c);
+    cs[(size_t)z * 2 * half + f] = (float)c;
+    cs[(size_t)z * 2 * half + half + f] = (float)s;
+    if (steps && f == 0) steps[z] = {0, base + z, {0, 0}};
+}
+
+extern "C" hipError_t sgk_rope_rows(const double *inv, uint32_t rope_dim, uint32_t base, uint32_t n, float *cs,
+                                    sgk_step *steps, hipStream_t s) {
+    const uint32_t half = rope_dim / 2;
+    if (!half || half > SGK_ROPE_HALF) return hipErrorInvalidValue;
+    if (!n) return hipSuccess;
+    rope_inv v = {};
+    for (uint32_t i = 0; i < half; i++) v.f[i] = inv[i];
+    const uint64_t blocks = ((uint64_t)n * half + TPB - 1) / TPB;
+    hipLaunchKernelGGL(k_rope_rows, dim3((uint32_t)blocks), dim3(TPB), 0, s, v, half, base, n, cs, steps);
+    return hipGetLastError();
 }
 
 // q_norm/k_norm + RoPE + f16 KV store. Workgroup (head, token): query heads
 // first, then kv heads.
 __global__ void __launch_bounds__(TPB) k_attn_prep(sgk_attn a, const float *qn, const float *kn,
-                                                   const float *cs_table, float eps) {
+                                                   const float *cs_table, uint32_t cs0, float eps) {
     __shared__ float red[4];
     __shared__ float buf[TPB];
     const uint32_t z = blockIdx.y, pos = a.steps[z].pos, t = threadIdx.x, b = blockIdx.x, hd = a.hd;
-    const float *cs = cs_table + (size_t)pos * a.rope_dim;
+    const float *cs = cs_table + (size_t)(pos - cs0) * a.rope_dim;
     const bool isq = b < a.n_heads;
     const uint32_t kh = b - a.n_heads;
-    float *row = (float *)a.q + (size_t)z * a.q_tok;
-    float *x = isq ? row + (size_t)b * a.q_stride : row + (size_t)a.n_heads * a.q_stride + (size_t)kh * hd;
+    const float *row = a.src + (size_t)z * a.src_tok;
+    const float *x = row + (isq ? (size_t)b * a.src_stride : (size_t)a.n_heads * a.src_stride + (size_t)kh * hd);
     const float *w = isq ? qn : kn;
     const float v = t < hd ? x[t] : 0.0f;
     const float ss = block_sum(v * v, red);
@@ -1185,20 +1216,21 @@ __global__ void __launch_bounds__(TPB) k_attn_prep(sgk_attn a, const float *qn, 
     else if (t < a.rope_dim) o = buf[t - half] * cs[t] + buf[t] * cs[t - half];
     if (t >= hd) return;
     if (isq) {
-        x[t] = o;
+        a.q[(size_t)z * a.q_tok + (size_t)b * a.q_stride + t] = o;
     } else {
         const size_t at = kv_at(a, pos, kh) + t;
-        const float *vraw = row + (size_t)a.n_heads * a.q_stride + (size_t)a.n_kv * hd + (size_t)kh * hd;
+        const float *vraw = row + (size_t)a.n_heads * a.src_stride + (size_t)a.n_kv * hd + (size_t)kh * hd;
         ((uint16_t *)a.kc)[at] = f2h(o);
         ((uint16_t *)a.vc)[at] = f2h(vraw[t]);
     }
 }
 
 extern "C" hipError_t sgk_attn_prep(const sgk_attn *a, const float *qn, const float *kn,
-                                    const float *cs_table, float eps, hipStream_t s) {
+                                    const float *cs_table, uint32_t cs0, float eps, hipStream_t s) {
     if (a->hd > TPB || !a->ntok) return a->ntok ? hipErrorInvalidValue : hipSuccess;
-    hipLaunchKernelGGL(k_attn_prep, dim3(a->n_heads + a->n_kv, a->ntok), dim3(TPB), 0, s, kv_resolved(a), qn, kn,
-                       cs_table, eps);
+    sgk_attn k = kv_resolved(a);
+    if (!k.src) { k.src = k.q; k.src_tok = k.q_tok; k.src_stride = k.q_stride; }
+    hipLaunchKernelGGL(k_attn_prep, dim3(a->n_heads + a->n_kv, a->ntok), dim3(TPB), 0, s, k, qn, kn, cs_table, cs0, eps);
     return hipGetLastError();
 }
 
@@ -2028,7 +2060,7 @@ __global__ void __launch_bounds__(TPB) k_attn_combine(sgk_attn a) {
     const float *mh = a.m + zoff + (size_t)h * ns, *sh = a.s + zoff + (size_t)h * ns;
     const float4 *acc = (const float4 *)(a.acc + (zoff + (size_t)h * ns) * HD);
     float *oh = a.out + (size_t)z * a.out_tok + (size_t)h * HD;
-    const float *gate = a.gate ? a.gate + (size_t)z * a.q_tok + (size_t)h * a.q_stride : NULL;
+    const float *gate = a.gate ? a.gate + (size_t)z * a.gate_tok + (size_t)h * a.gate_stride : NULL;
     // every load that does not depend on the merge weights goes out first:
     // this thread's first split's max and sum, and its first PFX rows of acc
     const uint32_t c = t % C4, kg = t / C4;
@@ -2348,7 +2380,7 @@ __global__ void __launch_bounds__(TPB * HW) k_attn_flash(sgk_attn a) {
     }
     // finish: o / s, sigmoid gate, store (lane: token li, dims 16n + 4lg + e)
     float *out = a.out + (size_t)zq * a.out_tok + (size_t)h * HD;
-    const float *gate = a.gate ? a.gate + (size_t)zq * a.q_tok + (size_t)h * a.q_stride : NULL;
+    const float *gate = a.gate ? a.gate + (size_t)zq * a.gate_tok + (size_t)h * a.gate_stride : NULL;
 #pragma unroll
     for (int n = 0; n < NNT; n++) {
         const uint32_t d0 = n * 16 + lg * 4;
@@ -2408,7 +2440,7 @@ extern "C" hipError_t sgk_attn_combine(const sgk_attn *a, hipStream_t s) {
     if (!a->n_heads || !a->ntok) return hipSuccess;
     if (!a->steps && a->n_splits > 1024) return hipErrorInvalidValue;
     dim3 grid(a->n_heads, a->ntok);
-#define HDCASE(H) case H: hipLaunchKernelGGL(k_attn_combine<H>, grid, dim3(TPB), 0, s, *a); break
+#define HDCASE(H) case H: hipLaunchKernelGGL(k_attn_combine<H>, grid, dim3(TPB), 0, s, kv_resolved(a)); break
     switch (a->hd) {
         HDCASE(16); HDCASE(32); HDCASE(64); HDCASE(128); HDCASE(256);
     default: return hipErrorInvalidValue;

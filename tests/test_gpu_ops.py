@@ -886,6 +886,29 @@ def test_attn_prefill_chunk_vs_oracle(gpu, nh, nkv, hd, rd, base, n):
     assert (np.abs(got_kv[0, base:].astype(np.float32) - Ko[base:]) <= ulp).all()
 
 
+@pytest.mark.parametrize("rd,base,n", [(2, 0, 1), (256, 70000, 3), (62, 131, 9)])
+def test_attn_chunk_rope_rows(gpu, rd, base, n):
+    """The chunk's RoPE rows (k_rope_rows): one frequency, as many as fit, and a
+    count that does not divide a workgroup; K against numpy's in float64 within
+    one f16 ulp (2^-10 of the value; values under 2^-14 have the subnormals'
+    spacing 2^-24), which a row, frequency or position off by one misses."""
+    nh, nkv, hd, theta, eps = 2, 1, 256, 1e6, 1e-6
+    rng = np.random.default_rng(rd + base)
+    inp = rng.standard_normal((n, 2 * nh * hd + 2 * nkv * hd)).astype(np.float32)
+    w = np.ones(2 * hd, np.float32)
+    kvb = gpu.buf(np.zeros(2 * (base + n) * hd, np.uint16))
+    gpu.attn_chunk(gpu.buf(inp.reshape(-1)), gpu.buf(w), kvb, gpu.buf(np.zeros(n * nh * hd, np.float32)),
+                   [nh, nkv, hd, rd, base, n, S.fbits(theta), S.fbits(eps)])
+    got = kvb.array.view(np.float16).reshape(2, base + n, hd)[0, base:].astype(np.float64)
+    k = inp[:, 2 * nh * hd:2 * nh * hd + hd].astype(np.float64)
+    k /= np.sqrt((k * k).mean(-1, keepdims=True) + eps)
+    ang = (base + np.arange(n))[:, None] * theta ** (-2.0 * np.arange(rd // 2) / rd)
+    a, b = k[:, :rd // 2].copy(), k[:, rd // 2:rd].copy()
+    k[:, :rd // 2] = a * np.cos(ang) - b * np.sin(ang)
+    k[:, rd // 2:rd] = a * np.sin(ang) + b * np.cos(ang)
+    assert (np.abs(got - k) <= np.maximum(np.abs(k) * 2.0 ** -10, 2.0 ** -24)).all()
+
+
 def test_attn_chunk_rejects_bad_shapes(gpu):
     """n_heads not a multiple of n_kv, head_dim 96, odd or oversize rope, an
     empty chunk, a chunk longer than its input rows, the cache aliasing the
