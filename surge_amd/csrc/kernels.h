@@ -86,6 +86,9 @@ typedef struct {
 } sgk_gemv;
 
 hipError_t sgk_gemv_launch(const sgk_gemv *a, hipStream_t s);
+/* y = W x (plain store) on a matrix of the file's 34-byte blocks, 2-byte
+ * aligned, without a repack; cols % 32 == 0, x 16-byte aligned. */
+hipError_t sgk_gemv_raw(const uint8_t *w, uint32_t rows, uint32_t cols, const float *x, float *y, hipStream_t s);
 
 /* Split Q8_0 blocks (34-byte) of a [rows, cols] matrix into the device layout
  * (qs [ld][cols] int8, d [ld][cols/32] f16 scales) and, when dt is not NULL,

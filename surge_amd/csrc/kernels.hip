@@ -540,6 +540,64 @@ __global__ void __launch_bounds__(TPB) k_gemv_ring(sgk_gemv a) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// Q8_0 GEMV on the file's 34-byte blocks (the one-call matvec: a matrix in
+// the caller's memory, used once, is not worth a repack into two planes).
+//
+// Bound by HBM, 34 bytes per 32 weights: lane l takes half blocks l, l+64, ...
+// of a row pair, 16 weights at 2-byte alignment (global loads of any width may
+// be unaligned on gfx950; a wave's 64 lanes cover 1088 consecutive bytes) and
+// the block's scale. RAW_U half blocks of both rows are in flight per lane, the
+// first ones requested before x is staged. Lanes, chunks and summation order
+// are k_gemv_q8's (k_repack_q8, then the GEMV on the planes, before: 18.2 + 5.4
+// us at 4096 x 4096, now 6.7; 94 MB at 5120 columns 127 + 18, now 27). Four half
+// blocks in flight instead of two took 80 registers and 8.3 and 33 us; x in the
+// chunked LDS layout 85 -> 89 us over 151936 x 2048.
+// ---------------------------------------------------------------------------
+#define RAW_U 2
+typedef uint32_t v4u_a2 __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ void raw_load(gemv_chunk<2> &ch, const uint8_t *w, uint32_t r0, uint32_t rows, size_t rb,
+                                         uint32_t nch, uint32_t c) {
+    const uint32_t cc = min(c, nch - 1);
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const uint8_t *p = w + (size_t)min(r0 + r, rows - 1) * rb + (size_t)(cc >> 1) * 34;
+        const v4u_a2 v = *(const v4u_a2 *)(p + 2 + 16 * (cc & 1));
+        ch.q[r] = make_uint4(v.x, v.y, v.z, v.w);
+        ch.d[r] = c < nch ? *(const uint16_t *)p : (uint16_t)0;
+    }
+}
+
+__global__ void __launch_bounds__(TPB) k_gemv_raw(sgk_gemv a, const uint8_t *w) {
+    extern __shared__ float xs[];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nch = a.cols >> 4;
+    const uint32_t ngroups = (a.rows + 1) / 2, gstride = gridDim.x * (TPB / 64);
+    const size_t rb = (size_t)(a.cols >> 5) * 34;
+    uint32_t g = blockIdx.x * (TPB / 64) + wave;
+    xstage<SGK_PRO_NONE, TPB, XK> st;
+    stage_issue<SGK_PRO_NONE, TPB, XK>(a, st);
+    gemv_chunk<2> ch[RAW_U];
+    const uint32_t gl = min(g, ngroups - 1);
+#pragma unroll
+    for (int u = 0; u < RAW_U; u++) raw_load(ch[u], w, gl * 2, a.rows, rb, nch, lane + 64 * u);
+    stage_finish<SGK_PRO_NONE, TPB, XK>(a, st, xs);
+    for (; g < ngroups; g += gstride) {
+        float acc[2] = {0.0f, 0.0f};
+        for (uint32_t c = lane;;) {
+#pragma unroll
+            for (int u = 0; u < RAW_U; u++) gemv_fma<2, false>(acc, ch[u], xs, min(c + 64 * u, nch - 1));
+            c += 64 * RAW_U;
+            const bool more = c - lane < nch;
+            // the row's next half blocks, or the next row pair's first
+            const uint32_t ng = more ? g : min(g + gstride, ngroups - 1), nc = more ? c : lane;
+#pragma unroll
+            for (int u = 0; u < RAW_U; u++) raw_load(ch[u], w, ng * 2, a.rows, rb, nch, nc + 64 * u);
+            if (!more) break;
+        }
+        gemv_finish<2, SGK_EPI_STORE>(a, acc, g * 2, lane, 1.0f);
+    }
+}
+
 // f32-weight GEMV (small test models only): one wave per row pair.
 template <int PRO, int EPI>
 __global__ void __launch_bounds__(TPB) k_gemv_f32(sgk_gemv a) {
@@ -932,6 +990,22 @@ extern "C" hipError_t sgk_gemv_launch(const sgk_gemv *a, hipStream_t s) {
     CASE(SGK_PRO_GATED, SGK_EPI_STORE);
 #undef CASE
     return hipErrorInvalidValue;
+}
+
+// y = W x on a matrix of 34-byte blocks (2-byte aligned), x 16-byte aligned.
+extern "C" hipError_t sgk_gemv_raw(const uint8_t *w, uint32_t rows, uint32_t cols, const float *x, float *y, hipStream_t s) {
+    if (((uintptr_t)x & 15) || ((uintptr_t)w & 1) || cols % 32) return hipErrorInvalidValue;
+    if (!rows || !cols) return hipSuccess;
+    sgk_gemv a = {};
+    a.rows = rows; a.cols = cols; a.x = x; a.y = y;
+    const size_t lds = (size_t)cols * 4;
+    hipError_t e = allow_lds((const void *)k_gemv_raw, lds);
+    if (e != hipSuccess) return e;
+    // resident workgroups only (VGPRs allow 8 a CU): each walks row pairs with a grid stride
+    const uint32_t per = min((uint32_t)(163840 / lds), 8u), groups = (rows + 1) / 2;
+    const uint32_t blocks = min((groups + 3) / 4, (uint32_t)device_cus() * per);
+    hipLaunchKernelGGL(k_gemv_raw, dim3(blocks), dim3(TPB), lds, s, a, w);
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------

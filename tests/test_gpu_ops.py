@@ -8,6 +8,8 @@ max|err|/max|want| and per element with an absolute floor of 1e-3*max|want|.
 The GPU accumulates in fp32 where the oracle uses double, so ~1e-6 is the
 expected error; 1e-3 is the acceptance bar.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -99,6 +101,28 @@ def test_gemv_q8_shapes(gpu, rows, cols):
     raw = q8_matrix(rng, rows, cols, sigma=1.0)
     x = rng.standard_normal(cols).astype(np.float32)
     assert_close(gpu_matvec_q8(gpu, raw, x, rows, cols), oracle_matvec_q8(raw, x, rows, cols))
+
+
+@pytest.mark.parametrize("rows,cols,off", [(1, 32, 2), (3, 96, 6), (2 * 8 * 1024 + 5, 2080, 0), (7, 40960, 14),
+                                           (9, 4128, 1)])
+def test_gemv_q8_on_blocks(gpu, rows, cols, off):
+    """The GEMV on 34-byte blocks where it can go wrong: one block, a row group
+    and a step cut short, more row groups than resident waves, the widest x the
+    LDS holds, and blocks off their natural alignment (an odd address takes the
+    repack): fp32 sums of cols terms against the oracle's doubles, rounding at
+    most 2^-24 a term and step, so 1e-5 of the largest |y| is far above it."""
+    rng = np.random.default_rng(rows + cols)
+    raw = q8_matrix(rng, rows, cols)
+    x = rng.standard_normal(cols).astype(np.float32)
+    held = gpu.buf(np.concatenate([np.zeros(off, np.uint8), raw]))
+    S.check(S.lib().sg_gpu_buf_upload(held.handle))
+    h = C.c_void_p()
+    S.check(S.lib().sg_gpu_wrap_device(gpu.handle, S.lib().sg_gpu_buf_device(held.handle) + off, raw.size, C.byref(h)))
+    xb, yb = gpu.buf(x), gpu.buf(np.zeros(rows, np.float32))
+    S.check(S.lib().sg_gpu_run_op(gpu.handle, b"k_matvec_q8", h, xb.handle, yb.handle, S.params([rows, cols])))
+    S.lib().sg_gpu_buf_free(h)
+    held.free()
+    assert_close(yb.array, oracle_matvec_q8(raw, x, rows, cols), 1e-5)
 
 
 def test_gemv_f32(gpu):
