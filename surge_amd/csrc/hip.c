@@ -746,6 +746,18 @@ sg_err sg_gpu_run_gdn_step(sg_gpu *g, void *in, void *w, void *state, void *out,
         return (sg_err){"gpu: gdn_step: buffers must not overlap"};
     void *ins[3] = {in, w, state}, *outs[2] = {state, out};
     if (sg_failed(e = push(ins, 3))) return e;
+    if (dv % SGK_GDN_BLOCKS == 0) {         /* on the tail itself; scratch: the row blocks' sums of squares */
+        void *ss;
+        if (sg_failed(e = scratch(g, (uint64_t)nv * SGK_GDN_BLOCKS * 4, &ss))) return e;
+        float *dst = DEV(state), *wp = DEV(w);
+        sgk_gdn d = {0};
+        d.in = DEV(in); d.z = (const float *)DEV(in) + cd; d.conv_w = wp; d.ssm_a = wp + cd * ks;
+        d.dt_bias = d.ssm_a + nv; d.norm_w = d.dt_bias + nv; d.ring = dst; d.S = dst + keep * cd;
+        d.n_k = nk; d.n_v = nv; d.dk = dk; d.dv = dv; d.conv_dim = (uint32_t)cd; d.ksize = ks;
+        d.tiled = p[5] != 0; d.neg_exp = p[6] != 0; d.out = DEV(out); d.eps = fbits(p[7]);
+        d.ss = ss; d.blocks = SGK_GDN_BLOCKS;
+        return finish(g, sgk_gdn_step_tail(&d, g->stream), outs, 2);
+    }
     /* scratch: the step descriptor, then the 4-slot ring. The step runs at
      * position 3, so the taps read slots 3-keep .. 2, which take the conv
      * tail's rows, and the input goes to slot 3. */

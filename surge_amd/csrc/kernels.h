@@ -224,6 +224,10 @@ typedef struct {
  * else SGK_GDN_BLOCKS per head, dv <= SGK_GDN_MAX_DV, RMSNormGated's per-head
  * factor applied by the out projection's SGK_PRO_GATED prologue). */
 hipError_t sgk_gdn_step(const sgk_gdn *a, hipStream_t s);
+/* The step on a caller's conv tail (ring = [ksize-1][conv_dim], oldest first,
+ * moved on in place; no step descriptor), RMSNormGated finished into out; dv a
+ * multiple of SGK_GDN_BLOCKS, ss scratch. */
+hipError_t sgk_gdn_step_tail(const sgk_gdn *a, hipStream_t s);
 
 /* The DeltaNet layer over a prefill chunk of ntok tokens (a->step holds the
  * chunk's descriptors, a->in the chunk's GEMM rows at in_stride, a->y the

@@ -2655,7 +2655,10 @@ __device__ __forceinline__ uint32_t rows_lane(uint32_t r) {   // a lane holding 
 // every block's readouts, so it is left to the output projection's gated
 // prologue: each block writes silu(z) * (y * w) of its rows and the sum of its
 // rows' squared readouts, with no synchronisation between blocks.
-template <int DK, int RW, int NB, int GDN_TPB>
+// TAIL: the conv's past inputs are the caller's tail, oldest first
+// (a.ring = [ksize-1][conv_dim]), which is only read here (k_gdn_finish moves
+// it on); no position is needed.
+template <int DK, int RW, int NB, int GDN_TPB, bool TAIL>
 __device__ __forceinline__ void gdn_step_body(const sgk_gdn &a, uint32_t h, uint32_t jb) {
     constexpr int GDN_NB = NB;
     constexpr int EPL = DK >= 64 ? DK / 64 : 1;
@@ -2668,7 +2671,7 @@ __device__ __forceinline__ void gdn_step_body(const sgk_gdn &a, uint32_t h, uint
     const uint32_t dk = DK, dv = a.dv, key_dim = a.n_k * dk, cd = a.conv_dim;
     const uint32_t rpb = (dv + GDN_NB - 1) / GDN_NB, jlo = jb * rpb, jhi = min(dv, jlo + rpb);
     const uint32_t hk = a.tiled ? h % a.n_k : h / (a.n_v / a.n_k);
-    const uint32_t pos = a.step->pos, keep = a.ksize - 1;
+    const uint32_t keep = a.ksize - 1, pos = TAIL ? keep : a.step->pos;   // TAIL: tap jj is row jj
     // The ring slot of the q/k channels is written by block 0 of the first
     // value head mapped to hk only (one writer per channel).
     const bool qk_writer = jb == 0 && (a.tiled ? h < a.n_k : (h % (a.n_v / a.n_k)) == 0);
@@ -2703,10 +2706,11 @@ __device__ __forceinline__ void gdn_step_body(const sgk_gdn &a, uint32_t h, uint
         cw.y = a.conv_w[(size_t)c * a.ksize + min(1u, keep)];
         cw.z = a.conv_w[(size_t)c * a.ksize + min(2u, keep)];
         cw.w = a.conv_w[(size_t)c * a.ksize + min(3u, keep)];
+        // a tail has keep rows (with none, the state behind it is read and not used)
         rs.x = a.ring[c];
-        rs.y = a.ring[(size_t)cd + c];
-        rs.z = a.ring[(size_t)2 * cd + c];
-        rs.w = a.ring[(size_t)3 * cd + c];
+        rs.y = a.ring[(size_t)(TAIL ? min(1u, max(keep, 1u) - 1) : 1) * cd + c];
+        rs.z = a.ring[(size_t)(TAIL ? min(2u, max(keep, 1u) - 1) : 2) * cd + c];
+        rs.w = TAIL ? 0.0f : a.ring[(size_t)3 * cd + c];
     };
     const uint32_t ch0 = chan(min(t, nch - 1)), ch1 = chan(min(t + GDN_TPB, nch - 1));
     conv_loads(cx0, cw0, rs0, ch0);
@@ -2745,7 +2749,7 @@ __device__ __forceinline__ void gdn_step_body(const sgk_gdn &a, uint32_t h, uint
         const float o = silu(acc);
         if (e < nch) {
             if (e < 2 * dk) qk[e] = o; else vv[e - 2 * dk] = o;
-            if (e >= 2 * dk || qk_writer) a.ring[(size_t)(pos & 3) * cd + c] = cx;
+            if (!TAIL && (e >= 2 * dk || qk_writer)) a.ring[(size_t)(pos & 3) * cd + c] = cx;
         }
     };
     // computed unconditionally (only the stores are guarded), so the second
@@ -2849,9 +2853,69 @@ __device__ __forceinline__ void gdn_step_body(const sgk_gdn &a, uint32_t h, uint
     if (t >= jlo && t < jhi) a.out[(size_t)h * dv + t] = silu(zj) * (ysh[t] * nwt);
 }
 
-template <int DK, int RW, int NB, int GDN_TPB>
+template <int DK, int RW, int NB, int GDN_TPB, bool TAIL = false>
 __global__ void __launch_bounds__(GDN_TPB) k_gdn_step(sgk_gdn a) {
-    gdn_step_body<DK, RW, NB, GDN_TPB>(a, blockIdx.x, blockIdx.y);
+    gdn_step_body<DK, RW, NB, GDN_TPB, TAIL>(a, blockIdx.x, blockIdx.y);
+}
+
+// A conv tail (oldest first, [keep][cd]) after ntok more inputs, in place: row
+// j takes the input of token ntok - keep + j, or the old row ntok + j while
+// that one is still inside the window (rows are read before they are written:
+// ntok + j > j).
+__device__ __forceinline__ void conv_tail(const float *in, uint32_t in_stride, float *tail, uint32_t ntok,
+                                          uint32_t cd, uint32_t keep, uint32_t ch) {
+    for (uint32_t j = 0; j < keep; j++)
+        tail[(size_t)j * cd + ch] = ntok + j < keep ? tail[(size_t)(ntok + j) * cd + ch]
+                                                    : in[(size_t)(ntok + j - keep) * in_stride + ch];
+}
+__global__ void k_conv_tail(const float *in, uint32_t in_stride, float *tail, uint32_t ntok, uint32_t cd, uint32_t keep) {
+    const uint32_t ch = blockIdx.x * TPB + threadIdx.x;
+    if (ch < cd) conv_tail(in, in_stride, tail, ntok, cd, keep, ch);
+}
+
+// What a step on the caller's tail leaves to do: each head's RMS factor from
+// its row blocks' sums of squares (added in block order, as the gated GEMV
+// prologue does) applied to its outputs, and the tail moved on by one input.
+// Thread i takes output i and channel i.
+__global__ void __launch_bounds__(TPB) k_gdn_finish(sgk_gdn a) {
+    const uint32_t i = blockIdx.x * TPB + threadIdx.x;
+    if (i < a.n_v * a.dv) {
+        const uint32_t h = i / a.dv;
+        float tot = 0.0f;
+#pragma unroll
+        for (uint32_t b = 0; b < SGK_GDN_BLOCKS; b++) tot += a.ss[h * SGK_GDN_BLOCKS + b];
+        a.out[i] *= 1.0f / sqrtf(tot / (float)a.dv + a.eps);
+    }
+    if (i < a.conv_dim) conv_tail((const float *)a.in, 0, (float *)a.ring, 1, a.conv_dim, a.ksize - 1, i);
+}
+
+// The step on a caller's conv tail: SGK_GDN_BLOCKS workgroups per head (dv a
+// multiple of that) and k_gdn_finish. Bound by latency, so by launches: the
+// ring form's one workgroup per head, with the descriptor copied in and the
+// tail copied to the ring and back around it, took 25.2 us a call at 16 heads
+// of 128 x 128 (step 7.4 us, three copies); this takes 18.4, some 10 of them
+// the launches and the wait.
+extern "C" hipError_t sgk_gdn_step_tail(const sgk_gdn *a, hipStream_t s) {
+    if (a->ksize < 1 || a->ksize > 4 || !a->n_k || a->n_v % a->n_k) return hipErrorInvalidValue;
+    if (!a->dv || a->dv % SGK_GDN_BLOCKS || a->dv > SGK_GDN_MAX_DV || !a->z || !a->out || !a->norm_w || !a->ss)
+        return hipErrorInvalidValue;
+    const uint32_t rpb = a->dv / SGK_GDN_BLOCKS, n = a->n_v * a->dv;
+    dim3 grid(a->n_v, SGK_GDN_BLOCKS);
+#define DKCASET(D) case D:                                                                                  \
+        if (rpb <= 8) hipLaunchKernelGGL((k_gdn_step<D, 2, SGK_GDN_BLOCKS, 256, true>), grid, dim3(256), 0, s, *a);        \
+        else if (rpb <= 16) hipLaunchKernelGGL((k_gdn_step<D, 4, SGK_GDN_BLOCKS, 256, true>), grid, dim3(256), 0, s, *a);  \
+        else if (rpb <= 32) hipLaunchKernelGGL((k_gdn_step<D, 8, SGK_GDN_BLOCKS, 256, true>), grid, dim3(256), 0, s, *a);  \
+        else hipLaunchKernelGGL((k_gdn_step<D, 16, SGK_GDN_BLOCKS, 256, true>), grid, dim3(256), 0, s, *a);                \
+        break
+    switch (a->dk) {
+        DKCASET(32); DKCASET(64); DKCASET(128); DKCASET(256);
+    default: return hipErrorInvalidValue;
+    }
+#undef DKCASET
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_gdn_finish, dim3((max(n, a->conv_dim) + TPB - 1) / TPB), dim3(TPB), 0, s, *a);
+    return hipGetLastError();
 }
 
 extern "C" hipError_t sgk_gdn_step(const sgk_gdn *a, hipStream_t s) {

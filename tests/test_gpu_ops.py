@@ -509,6 +509,15 @@ def test_gdn_prefill_chunk_vs_oracle(gpu, nv, nk, dk, dv, ks, tiled, n1, n2):
         ob.free()
 
 
+@pytest.mark.parametrize("nv,nk,dk,dv,ks,tiled", [(2, 2, 32, 4, 1, True), (3, 1, 64, 12, 3, False), (4, 2, 256, 72, 2, True),
+                                                  (2, 1, 32, 5, 4, True), (6, 3, 64, 124, 4, True)])
+def test_gdn_step_on_tail_edges(gpu, nv, nk, dk, dv, ks, tiled):
+    """The step on the caller's tail where it can go wrong: no tail at all, one
+    and two rows, one row and a part-filled wave per block, and a head_v_dim the
+    four blocks do not divide (the ring form with its copies)."""
+    test_gdn_decode_step_vs_oracle(gpu, nv, nk, dk, dv, ks, tiled)
+
+
 def test_gdn_step_rejects_bad_shapes(gpu):
     b = gpu.buf(np.zeros(1 << 16, np.float32))
     o = gpu.buf(np.zeros(1 << 12, np.float32))
