@@ -792,8 +792,8 @@ sg_err sg_gpu_run_gdn_step(sg_gpu *g, void *in, void *w, void *state, void *out,
  *         updated in place;
  *   out   [n][value_dim].
  * p: [0]=dk [1]=dv [2]=n_v [3]=n_k [4]=ksize [5]=flags: bit 0 tiled, bit 1
- * ssm_a is -exp(A_log), bits 2-3 the first position mod 4 (the ring slot the
- * chunk starts at) [6]=n [7]=eps bits. */
+ * ssm_a is -exp(A_log), bits 2-3 the first position mod 4 (the conv reads and
+ * moves the tail itself, so nothing depends on it) [6]=n [7]=eps bits. */
 sg_err sg_gpu_run_gdn_chunk(sg_gpu *g, void *in, void *w, void *state, void *out, const uint32_t p[8]) {
     if (!g || !in || !w || !state || !out || !p) return (sg_err){"gpu: gdn_chunk got a NULL argument"};
     const uint32_t dk = p[0], dv = p[1], nv = p[2], nk = p[3], ks = p[4], n = p[6];
@@ -811,39 +811,21 @@ sg_err sg_gpu_run_gdn_chunk(sg_gpu *g, void *in, void *w, void *state, void *out
         return (sg_err){"gpu: gdn_chunk: buffers must not overlap"};
     void *ins[3] = {in, w, state}, *outs[2] = {state, out};
     if (sg_failed(e = push(ins, 3))) return e;
-    /* scratch: the chunk's step descriptors, the 4-slot ring, the conv
-     * output, the scan readouts and the scan workspace */
-    const uint64_t sb = ((uint64_t)n * sizeof(sgk_step) + 255) / 256 * 256, rb = 4 * cd * 4, cb = (uint64_t)n * cd * 4,
-                   yb = (uint64_t)n * vd * 4, wsb = (uint64_t)sgk_delta_ws_floats(nv, n) * 4;
+    /* scratch: the conv output, the scan readouts and the scan workspace */
+    const uint64_t cb = (uint64_t)n * cd * 4, yb = (uint64_t)n * vd * 4, wsb = (uint64_t)sgk_delta_ws_floats(nv, n) * 4;
     void *t;
-    if (sg_failed(e = scratch(g, sb + rb + cb + yb + wsb, &t))) return e;
-    const uint32_t pos0 = 4 + ((p[5] >> 2) & 3);
-    sgk_step *st = calloc(n, sizeof *st);
-    if (!st) return (sg_err){"gpu: gdn_chunk: out of host memory"};
-    for (uint32_t z = 0; z < n; z++) st[z].pos = pos0 + z;
+    if (sg_failed(e = scratch(g, cb + yb + wsb, &t))) return e;
     hipStream_t s = g->stream;
-    hipError_t he = hipMemcpyAsync(t, st, n * sizeof *st, hipMemcpyHostToDevice, s);
-    if (he == hipSuccess) he = hipStreamSynchronize(s);
-    free(st);
-    HIPCHK(he, "gdn_chunk descriptors");
-    float *ring = (float *)((char *)t + sb), *conv = ring + 4 * cd, *y = conv + (uint64_t)n * cd, *ws = y + (uint64_t)n * vd;
+    float *conv = t, *y = conv + (uint64_t)n * cd, *ws = y + (uint64_t)n * vd;
     float *dst = DEV(state), *wp = DEV(w);
-    /* the tail's row j is the input of position pos0 - keep + j */
-    for (uint64_t j = 0; j < keep; j++)
-        HIPCHK(hipMemcpyAsync(ring + ((pos0 - keep + j) & 3) * cd, dst + j * cd, cd * 4, hipMemcpyDeviceToDevice, s),
-               "conv tail in");
     sgk_gdn d = {0};
-    d.in = DEV(in); d.conv_w = wp; d.ssm_a = wp + cd * ks; d.dt_bias = d.ssm_a + nv; d.ring = ring;
-    d.S = dst + keep * cd; d.y = y; d.step = t; d.n_k = nk; d.n_v = nv; d.dk = dk; d.dv = dv;
+    d.in = DEV(in); d.conv_w = wp; d.ssm_a = wp + cd * ks; d.dt_bias = d.ssm_a + nv; d.ring = dst;
+    d.S = dst + keep * cd; d.y = y; d.n_k = nk; d.n_v = nv; d.dk = dk; d.dv = dv;
     d.conv_dim = (uint32_t)cd; d.ksize = ks; d.tiled = p[5] & 1; d.neg_exp = (p[5] >> 1) & 1;
-    he = sgk_gdn_chunk(&d, conv, (uint32_t)row, n, ws, s);
+    hipError_t he = sgk_gdn_chunk(&d, conv, (uint32_t)row, n, ws, s);
     if (he == hipSuccess)
         he = sgk_rmsnorm_gated_rows(y, (const float *)DEV(in) + cd, (uint32_t)row, d.ssm_a + 2 * nv, DEV(out), dv, nv, n,
                                     fbits(p[7]), s);
-    /* the new tail: the inputs of the last keep positions, which the ring
-     * holds (positions before the chunk kept their slots) */
-    for (uint64_t j = 0; he == hipSuccess && j < keep; j++)
-        he = hipMemcpyAsync(dst + j * cd, ring + ((pos0 + n - keep + j) & 3) * cd, cd * 4, hipMemcpyDeviceToDevice, s);
     return finish(g, he, outs, 2);
 }
 

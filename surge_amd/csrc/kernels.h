@@ -233,7 +233,8 @@ hipError_t sgk_gdn_step_tail(const sgk_gdn *a, hipStream_t s);
  * chunk's descriptors, a->in the chunk's GEMM rows at in_stride, a->y the
  * readouts [ntok][value_dim]): conv scan into conv_out [ntok][conv_dim], q/k
  * norms, then the delta-rule scan with S in registers. Same arithmetic as
- * sgk_gdn_step, token by token. */
+ * sgk_gdn_step, token by token. With a->step NULL, a->ring is a caller's conv
+ * tail [ksize-1][conv_dim], oldest first, moved on in place. */
 hipError_t sgk_gdn_chunk(const sgk_gdn *a, float *conv_out, uint32_t in_stride, uint32_t ntok,
                          float *ws, hipStream_t s);
 /* The delta-rule scan alone: qkv rows [ntok][a->conv_dim] hold normalised

@@ -109,11 +109,12 @@ __device__ __forceinline__ uint4 ldnt(const uint4 *p) {
 __device__ __forceinline__ float h2f(uint16_t h) { return __half2float(__ushort_as_half(h)); }
 __device__ __forceinline__ uint16_t f2h(float f) { return __half_as_ushort(__float2half_rn(f)); }
 
-// sigmoid split on the sign so exp never overflows (ref.c:127-134).
+// sigmoid split on the sign so exp never overflows (ref.c:127-134): 1 / (1 + e)
+// or e / (1 + e) with e = exp(-|x|), chosen by the numerator so that a wave of
+// both signs runs one exp and one division, not two of each.
 __device__ __forceinline__ float sigm(float x) {
-    if (x >= 0.0f) return 1.0f / (1.0f + expf(-x));
-    float e = expf(x);
-    return e / (1.0f + e);
+    const float e = expf(-fabsf(x));
+    return (x >= 0.0f ? 1.0f : e) / (1.0f + e);
 }
 __device__ __forceinline__ float silu(float x) { return x * sigm(x); }
 // max(x,0) + log1p(e^-|x|) (ref.c:136-142).
@@ -2868,10 +2869,6 @@ __device__ __forceinline__ void conv_tail(const float *in, uint32_t in_stride, f
         tail[(size_t)j * cd + ch] = ntok + j < keep ? tail[(size_t)(ntok + j) * cd + ch]
                                                     : in[(size_t)(ntok + j - keep) * in_stride + ch];
 }
-__global__ void k_conv_tail(const float *in, uint32_t in_stride, float *tail, uint32_t ntok, uint32_t cd, uint32_t keep) {
-    const uint32_t ch = blockIdx.x * TPB + threadIdx.x;
-    if (ch < cd) conv_tail(in, in_stride, tail, ntok, cd, keep, ch);
-}
 
 // What a step on the caller's tail leaves to do: each head's RMS factor from
 // its row blocks' sums of squares (added in block order, as the gated GEMV
@@ -3053,31 +3050,41 @@ extern "C" hipError_t sgk_rmsnorm_gated(const float *y, const float *z, const fl
 // RMS and scale before they are written: each wave sums its squares with
 // wave_sum, and a head's waves are added in block_sum's order (the same
 // per-lane values in the same lanes, so the same bits as the separate pass).
+// TAIL: the positions before the chunk are a caller's tail instead ([ksize-1]
+// [cd], oldest first; k_conv_tail moves it on afterwards).
+// CC tokens per thread: 16 (three inputs re-read per sixteen), or 4 while that
+// leaves most of the chip without a workgroup (a thread's loads, its 16 SiLUs
+// and a q/k wave's 16 sums are one serial chain: 45 tokens of 6144 channels 9.5 -> 5.2 us). 512 tokens of
+// 10240 channels: 16.4 us (19.6 with two exps and divisions per SiLU), its 42 MB
+// at 2.6 TB/s, the VALU as busy as the loads.
 #define CC_TOK 16
+template <bool TAIL, int CC>
 __global__ void __launch_bounds__(TPB) k_conv_chunk(const float *in, uint32_t in_stride, const float *conv_w,
                                                     const float *ring, float *out, const sgk_step *steps,
                                                     uint32_t ntok, uint32_t cd, uint32_t ksize, uint32_t qk_end,
                                                     uint32_t hw) {
-    __shared__ float red[4][CC_TOK];
-    const uint32_t ch = blockIdx.x * TPB + threadIdx.x, z0 = blockIdx.y * CC_TOK;
+    __shared__ float red[4][CC];
+    const uint32_t ch = blockIdx.x * TPB + threadIdx.x, z0 = blockIdx.y * CC;
     const bool live = ch < cd;
-    const uint32_t keep = ksize - 1, pos0 = steps[0].pos;
-    float o[CC_TOK];
+    const uint32_t keep = ksize - 1, pos0 = TAIL ? 0 : steps[0].pos;
+    float o[CC];
     if (live) {
-        float w[4], x[CC_TOK + 3];
+        float w[4], x[CC + 3];
 #pragma unroll
         for (uint32_t j = 0; j < 4; j++) w[j] = conv_w[(size_t)ch * ksize + min(j, keep)];
         // x[3 + i] = input of token z0 + i; x[0..2] = the three before z0
 #pragma unroll
-        for (int i = 0; i < CC_TOK + 3; i++) {
+        for (int i = 0; i < CC + 3; i++) {
             const int z = (int)z0 + i - 3;
             const uint32_t zc = (uint32_t)min(max(z, 0), (int)ntok - 1);
-            const float vi = in[(size_t)zc * in_stride + ch];
-            const float vr = ring[(size_t)((pos0 + 4 + (uint32_t)min(z, 0)) & 3) * cd + ch];
-            x[i] = z < 0 ? vr : vi;
+            x[i] = in[(size_t)zc * in_stride + ch];
+            if (i < 3 && z0 == 0) {      // z < 0; no tail row keep + z (z < -keep): not used
+                const uint32_t r = TAIL ? (uint32_t)max((int)keep + z, 0) : (pos0 + 4 + (uint32_t)z) & 3;
+                x[i] = ring[(size_t)r * cd + ch];
+            }
         }
 #pragma unroll
-        for (int i = 0; i < CC_TOK; i++) {
+        for (int i = 0; i < CC; i++) {
             float acc = 0.0f;
 #pragma unroll
             for (uint32_t jj = 0; jj < 3; jj++)
@@ -3088,28 +3095,28 @@ __global__ void __launch_bounds__(TPB) k_conv_chunk(const float *in, uint32_t in
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < CC_TOK; i++) o[i] = 0.0f;
+        for (int i = 0; i < CC; i++) o[i] = 0.0f;
     }
     if (hw && blockIdx.x * TPB < qk_end) {
         const uint32_t w = threadIdx.x >> 6;
-        float ss[CC_TOK];
+        float ss[CC];
 #pragma unroll
-        for (int i = 0; i < CC_TOK; i++) ss[i] = wave_sum(fmaf(o[i], o[i], 0.0f));
+        for (int i = 0; i < CC; i++) ss[i] = wave_sum(fmaf(o[i], o[i], 0.0f));
         if (hw > 1) {
             if ((threadIdx.x & 63) == 0)
 #pragma unroll
-                for (int i = 0; i < CC_TOK; i++) red[w][i] = ss[i];
+                for (int i = 0; i < CC; i++) red[w][i] = ss[i];
             __syncthreads();
             // block_sum's (r0 + r1) + (r2 + r3) with the other head's waves at zero
             const uint32_t w0 = w & 2;
 #pragma unroll
-            for (int i = 0; i < CC_TOK; i++) ss[i] = red[w0][i] + red[w0 + 1][i];
+            for (int i = 0; i < CC; i++) ss[i] = red[w0][i] + red[w0 + 1][i];
         }
         if (ch < qk_end) {
             const float dk = (float)(64 * hw);
             const float sc = ch < qk_end / 2 ? 1.0f / dk : 1.0f / sqrtf(dk);
 #pragma unroll
-            for (int i = 0; i < CC_TOK; i++) {
+            for (int i = 0; i < CC; i++) {
                 const float r = 1.0f / sqrtf(ss[i] / dk + 1e-6f);
                 o[i] = (o[i] * r) * sc;
             }
@@ -3117,19 +3124,27 @@ __global__ void __launch_bounds__(TPB) k_conv_chunk(const float *in, uint32_t in
     }
     if (live)
 #pragma unroll
-        for (int i = 0; i < CC_TOK; i++)
+        for (int i = 0; i < CC; i++)
             if (z0 + i < ntok) out[(size_t)(z0 + i) * cd + ch] = o[i];
 }
 
-// The ring after a chunk: slot p % 4 = input of position p for the chunk's
-// last min(ntok, 4) positions (older slots keep their values).
-__global__ void k_conv_ring(const float *in, uint32_t in_stride, float *ring, const sgk_step *steps,
-                            uint32_t ntok, uint32_t cd) {
-    const uint32_t ch = blockIdx.x * TPB + threadIdx.x;
-    if (ch >= cd) return;
-    const uint32_t pos0 = steps[0].pos;
+// The conv's past inputs after a chunk, channel ch: slot p % 4 of the ring =
+// input of position p for the chunk's last min(ntok, 4) positions (older slots
+// keep their values), or the caller's tail moved on.
+__device__ __forceinline__ void conv_window(const sgk_gdn &a, uint32_t in_stride, uint32_t ntok, uint32_t ch) {
+    const float *in = (const float *)a.in;
+    float *ring = (float *)a.ring;
+    if (!a.step) {
+        conv_tail(in, in_stride, ring, ntok, a.conv_dim, a.ksize - 1, ch);
+        return;
+    }
+    const uint32_t pos0 = a.step[0].pos;
     for (uint32_t z = ntok > 4 ? ntok - 4 : 0; z < ntok; z++)
-        ring[(size_t)((pos0 + z) & 3) * cd + ch] = in[(size_t)z * in_stride + ch];
+        ring[(size_t)((pos0 + z) & 3) * a.conv_dim + ch] = in[(size_t)z * in_stride + ch];
+}
+__global__ void k_conv_window(sgk_gdn a, uint32_t in_stride, uint32_t ntok) {
+    const uint32_t ch = blockIdx.x * TPB + threadIdx.x;
+    if (ch < a.conv_dim) conv_window(a, in_stride, ntok, ch);
 }
 
 // q and k of every key head of every token: RMS (eps 1e-6, no weight), then
@@ -3298,6 +3313,64 @@ __global__ void k_rmsnorm_gated_rows(const float *y, const float *zsrc, uint32_t
     for (uint32_t j = lane; j < dv; j += 64) oh[j] = silu(zh[j]) * ((yh[j] * r) * w[j]);
 }
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+// Element offset of X[n][k] in a product's bf16 hi | lo split (laid out per
+// Q8_0 block, see k_split_bf16), and four values put there.
+__device__ __forceinline__ size_t xs_at(uint32_t N, uint32_t n, uint32_t k) {
+    return ((size_t)(k >> 5) * N + n) * 64 + (k & 31);
+}
+__device__ __forceinline__ void xs_put4(uint16_t *xs, uint32_t N, uint32_t n, uint32_t k, const float (&v)[4]) {
+    const bf16x2 h01 = {(__bf16)v[0], (__bf16)v[1]}, h23 = {(__bf16)v[2], (__bf16)v[3]};
+    const bf16x2 l01 = {(__bf16)(v[0] - (float)h01[0]), (__bf16)(v[1] - (float)h01[1])};
+    const bf16x2 l23 = {(__bf16)(v[2] - (float)h23[0]), (__bf16)(v[3] - (float)h23[1])};
+    uint16_t *o = xs + xs_at(N, n, k);
+    *(uint2 *)o = make_uint2(__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23));
+    *(uint2 *)(o + 32) = make_uint2(__builtin_bit_cast(uint32_t, l01), __builtin_bit_cast(uint32_t, l23));
+}
+
+// The same for dv 64, 128 or 256 with 16-byte aligned rows: dv / 4 lanes per
+// head, four elements each. Bound by memory (38 MB at 512 tokens of 48 heads of 128): 8.4
+// us; the scalar form's 4-byte loads took 11.2, and 12.7 with 2-byte stores
+// into a split (8.6 now). XS: out is the next product's bf16 hi | lo split.
+template <uint32_t DV, bool XS>
+__global__ void __launch_bounds__(TPB) k_rmsnorm_gated_v4(const float *y, const float *zsrc, uint32_t z_stride,
+                                                          const float *w, void *out, uint32_t N, uint32_t n_v, float eps) {
+    constexpr uint32_t LPH = DV / 4;
+    const uint32_t e = blockIdx.x * TPB + threadIdx.x, h = e / LPH, c = e % LPH * 4, z = blockIdx.y;
+    const bool live = h < n_v;                  // n_v * LPH need not fill the last workgroup
+    const uint32_t hh = live ? h : n_v - 1;
+    const float4 v = *(const float4 *)(y + ((size_t)z * n_v + hh) * DV + c);
+    const float4 g = *(const float4 *)(zsrc + (size_t)z * z_stride + (size_t)hh * DV + c);
+    const float4 wv = *(const float4 *)(w + c);
+    float ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w)));
+    ss += lane_xor1(ss);
+    ss += lane_xor2(ss);
+    ss += lane_mir8(ss);
+    ss += lane_xor8(ss);
+    if (LPH > 16) ss += lane_xor16(ss);
+    if (LPH > 32) ss += lane_xor32(ss);
+    if (!live) return;
+    const float r = 1.0f / sqrtf(ss / (float)DV + eps);
+    const float o[4] = {silu(g.x) * ((v.x * r) * wv.x), silu(g.y) * ((v.y * r) * wv.y), silu(g.z) * ((v.z * r) * wv.z),
+                        silu(g.w) * ((v.w * r) * wv.w)};
+    if (XS) xs_put4((uint16_t *)out, N, z, h * DV + c, o);
+    else *(float4 *)((float *)out + ((size_t)z * n_v + h) * DV + c) = make_float4(o[0], o[1], o[2], o[3]);
+}
+// Whether the float4 form takes these rows.
+static bool norm_v4(const float *y, const float *z, uint32_t z_stride, const float *w, const void *out, uint32_t dv) {
+    return (dv == 64 || dv == 128 || dv == 256) && z_stride % 4 == 0 &&
+           !(((uintptr_t)y | (uintptr_t)z | (uintptr_t)w | (uintptr_t)out) & 15);
+}
+template <bool XS>
+static hipError_t norm_v4_launch(const float *y, const float *z, uint32_t z_stride, const float *w, void *out, uint32_t N,
+                                 uint32_t dv, uint32_t n_v, uint32_t ntok, float eps, hipStream_t s) {
+    const dim3 grid((n_v * (dv / 4) + TPB - 1) / TPB, ntok);
+    auto kern = dv == 64 ? k_rmsnorm_gated_v4<64, XS> : dv == 128 ? k_rmsnorm_gated_v4<128, XS> : k_rmsnorm_gated_v4<256, XS>;
+    hipLaunchKernelGGL(kern, grid, dim3(TPB), 0, s, y, z, z_stride, w, out, N, n_v, eps);
+    return hipGetLastError();
+}
+
 __global__ void k_embed_rows(const int8_t *qs, const uint16_t *d, const float *wf, uint32_t hidden,
                              const sgk_step *steps, float *X) {
     const uint32_t i = blockIdx.x * TPB + threadIdx.x, z = blockIdx.y;
@@ -3350,7 +3423,15 @@ __global__ void __launch_bounds__(TPB) k_dm_prep(sgk_gdn a, const float *qkv, ui
     __shared__ __align__(16) float Tl[TPB / 64][DM_T][DM_T];
     __shared__ float dl[TPB / 64][DM_T], bl[TPB / 64][DM_T];
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, s = lane >> 4;
-    const uint32_t nblk = (ntok + DM_T - 1) / DM_T, c = blockIdx.x * (TPB / 64) + wv, h = blockIdx.y;
+    const uint32_t nblk = (ntok + DM_T - 1) / DM_T;
+    // the workgroups past the blocks (one per head, if launched) move the conv's
+    // window on: its last reader was the conv, and a launch of its own took 4.7 us
+    if (blockIdx.x * (TPB / 64) >= nblk) {
+        for (uint32_t ch = blockIdx.y * TPB + threadIdx.x; ch < a.conv_dim; ch += gridDim.y * TPB)
+            conv_window(a, in_stride, ntok, ch);
+        return;
+    }
+    const uint32_t c = blockIdx.x * (TPB / 64) + wv, h = blockIdx.y;
     const bool live = c < nblk;                 // a wave past the last block computes block nblk-1, stores nothing
     const uint32_t cb = live ? c : nblk - 1, z0 = cb * DM_T, n = min((uint32_t)DM_T, ntok - z0);
     const uint32_t hk = a.tiled ? h % a.n_k : h / (a.n_v / a.n_k), key_dim = a.n_k * DK;
@@ -3641,6 +3722,9 @@ extern "C" uint64_t sgk_delta_ws_floats(uint32_t n_v, uint32_t ntok) {
     return (uint64_t)n_v * ((ntok + DM_T - 1) / DM_T) * DM_WS;
 }
 
+// window: also move the conv's past inputs on (conv_window), after the conv
+static hipError_t delta_scan(const sgk_gdn *a, const float *qkv, uint32_t in_stride, uint32_t ntok, const float *gates,
+                             float *ws, bool window, hipStream_t s);
 extern "C" hipError_t sgk_gdn_chunk(const sgk_gdn *a, float *conv_out, uint32_t in_stride, uint32_t ntok,
                                     float *ws, hipStream_t s) {
     if (!ntok) return hipSuccess;
@@ -3649,27 +3733,37 @@ extern "C" hipError_t sgk_gdn_chunk(const sgk_gdn *a, float *conv_out, uint32_t 
     const uint32_t hw = a->dk == 64 ? 1 : a->dk == 128 ? 2 : 0;
     const uint32_t qk_end = 2 * a->n_k * a->dk;
     if (qk_end > a->conv_dim) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_conv_chunk, dim3((a->conv_dim + TPB - 1) / TPB, (ntok + CC_TOK - 1) / CC_TOK), dim3(TPB), 0, s,
-                       a->in, in_stride, a->conv_w, a->ring, conv_out, a->step, ntok, a->conv_dim, a->ksize,
-                       hw ? qk_end : 0u, hw);
-    hipLaunchKernelGGL(k_conv_ring, dim3((a->conv_dim + TPB - 1) / TPB), dim3(TPB), 0, s, a->in, in_stride, a->ring,
-                       a->step, ntok, a->conv_dim);
+    const uint32_t cg = (a->conv_dim + TPB - 1) / TPB;
+    const bool few = (uint64_t)cg * ((ntok + CC_TOK - 1) / CC_TOK) < 2 * (uint64_t)device_cus();
+#define CONV(T, C) hipLaunchKernelGGL((k_conv_chunk<T, C>), dim3(cg, (ntok + (C) - 1) / (C)), dim3(TPB), 0, s, a->in, in_stride, \
+                                      a->conv_w, a->ring, conv_out, a->step, ntok, a->conv_dim, a->ksize, hw ? qk_end : 0u, hw)
+    if (a->step) { if (few) CONV(false, 4); else CONV(false, CC_TOK); }
+    else { if (few) CONV(true, 4); else CONV(true, CC_TOK); }
+#undef CONV
     if (!hw)
         hipLaunchKernelGGL(k_qk_norm_chunk, dim3(2 * a->n_k, ntok), dim3(TPB), 0, s, conv_out, a->conv_dim, a->n_k,
                            a->dk);
-    return sgk_delta_scan(a, conv_out, in_stride, ntok, NULL, ws, s);
+    return delta_scan(a, conv_out, in_stride, ntok, NULL, ws, true, s);
 }
 
 extern "C" hipError_t sgk_delta_scan(const sgk_gdn *a, const float *qkv, uint32_t in_stride, uint32_t ntok,
                                      const float *gates, float *ws, hipStream_t s) {
+    return delta_scan(a, qkv, in_stride, ntok, gates, ws, false, s);
+}
+
+static hipError_t delta_scan(const sgk_gdn *a, const float *qkv, uint32_t in_stride, uint32_t ntok, const float *gates,
+                             float *ws, bool window, hipStream_t s) {
     if (!ntok || !a->n_v || !a->dv) return hipSuccess;
     const int mode = ws && (a->dk == 64 || a->dk == 128) ? scan_mode() : SCAN_SEQ;
-    if (mode == SCAN_MFMA && a->dv % DM_T == 0) {
+    const bool mfma = mode == SCAN_MFMA && a->dv % DM_T == 0;
+    if (window && !mfma)
+        hipLaunchKernelGGL(k_conv_window, dim3((a->conv_dim + TPB - 1) / TPB), dim3(TPB), 0, s, *a, in_stride, ntok);
+    if (mfma) {
         // W', M, g, rho of every (head, 16-token block), then each head's
         // blocks in order per 16 value rows
         const uint32_t nblk = (ntok + DM_T - 1) / DM_T;
 #define DML(D) do {                                                                                                   \
-            hipLaunchKernelGGL((k_dm_prep<D>), dim3((nblk + TPB / 64 - 1) / (TPB / 64), a->n_v), dim3(TPB), 0, s, *a, qkv, \
+            hipLaunchKernelGGL((k_dm_prep<D>), dim3((nblk + TPB / 64 - 1) / (TPB / 64) + window, a->n_v), dim3(TPB), 0, s, *a, qkv, \
                                in_stride, ntok, gates, ws);                                                          \
             hipLaunchKernelGGL((k_dm_scan<D>), dim3(a->n_v, a->dv / DM_T), dim3(DM_TPB), 0, s, *a, qkv, ntok, ws); } while (0)
         if (a->dk == 64) DML(64); else DML(128);
@@ -3748,6 +3842,7 @@ extern "C" hipError_t sgk_rmsnorm_gated_rows(const float *y, const float *z, uin
                                              float *out, uint32_t dv, uint32_t n_v, uint32_t ntok, float eps,
                                              hipStream_t s) {
     if (!ntok || !n_v) return hipSuccess;
+    if (norm_v4(y, z, z_stride, w, out, dv)) return norm_v4_launch<false>(y, z, z_stride, w, out, 0, dv, n_v, ntok, eps, s);
     hipLaunchKernelGGL(k_rmsnorm_gated_rows, dim3((n_v + 3) / 4, ntok), dim3(TPB), 0, s, y, z, z_stride, w, out,
                        dv, n_v, eps);
     return hipGetLastError();
@@ -3854,16 +3949,11 @@ extern "C" hipError_t sgk_step_advance(sgk_step *step, uint32_t *hist, hipStream
 // B[k][j] in lane j + 16*(k/8); D[i][j] in lane j + 16*(i/4), element i%4.
 // ---------------------------------------------------------------------------
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
 // X [N][ldx] f32 -> bf16 hi and lo = x - hi (both round-to-nearest-even),
 // laid out per Q8_0 block: the 64 bf16 of block b of token n, hi (32) then lo
 // (32), at xs + (b*N + n)*64, so a K step of the GEMM reads one contiguous
 // 128-byte line per token (K % 32 == 0, ldx % 4 == 0, X 16-byte aligned).
-__device__ __forceinline__ size_t xs_at(uint32_t N, uint32_t n, uint32_t k) {
-    return ((size_t)(k >> 5) * N + n) * 64 + (k & 31);
-}
+
 // one value of X into the split: hi = bf16(v), lo = bf16(v - hi), as k_split_bf16 rounds them
 __device__ __forceinline__ void xs_put(uint16_t *xs, uint32_t N, uint32_t n, uint32_t k, float v) {
     const __bf16 hi = (__bf16)v, lo = (__bf16)(v - (float)hi);
@@ -3914,6 +4004,7 @@ extern "C" hipError_t sgk_rmsnorm_gated_split(const float *y, const float *z, ui
                                               hipStream_t s) {
     if (!ntok || !n_v) return hipSuccess;
     if (((uint64_t)n_v * dv) % 32 || ((uintptr_t)xs & 15)) return hipErrorInvalidValue;
+    if (norm_v4(y, z, z_stride, w, xs, dv)) return norm_v4_launch<true>(y, z, z_stride, w, xs, ntok, dv, n_v, ntok, eps, s);
     hipLaunchKernelGGL(k_rmsnorm_gated_split, dim3((n_v + 3) / 4, ntok), dim3(TPB), 0, s, y, z, z_stride, w, xs, ntok,
                        dv, n_v, eps);
     return hipGetLastError();

@@ -518,6 +518,15 @@ def test_gdn_step_on_tail_edges(gpu, nv, nk, dk, dv, ks, tiled):
     test_gdn_decode_step_vs_oracle(gpu, nv, nk, dk, dv, ks, tiled)
 
 
+@pytest.mark.parametrize("nv,nk,dk,dv,ks,tiled,n1,n2", [(48, 16, 128, 128, 4, True, 215, 1), (2, 1, 64, 64, 1, True, 3, 2),
+                                                        (3, 3, 128, 256, 3, True, 1, 17)])
+def test_gdn_chunk_forms(gpu, nv, nk, dk, dv, ks, tiled, n1, n2):
+    """The chunk conv with sixteen tokens per thread and with four, no tail, a
+    chunk shorter than the tail (old rows stay), and the float4 norm with rows
+    that do not fill a workgroup."""
+    test_gdn_prefill_chunk_vs_oracle(gpu, nv, nk, dk, dv, ks, tiled, n1, n2)
+
+
 def test_gdn_step_rejects_bad_shapes(gpu):
     b = gpu.buf(np.zeros(1 << 16, np.float32))
     o = gpu.buf(np.zeros(1 << 12, np.float32))
