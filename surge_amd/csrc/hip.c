@@ -118,7 +118,8 @@ struct sg_gpu {
     float *pf_X, *pf_Xn, *pf_IN, *pf_CONV, *pf_Y, *pf_G, *pf_CTX, *pf_FF, *pf_m, *pf_s, *pf_acc;
     uint16_t *pf_XS;        /* the prefill GEMMs' X split into bf16 hi | lo */
     uint16_t *pf_XS2;       /* a second split: gate/up writes the down projection's into it */
-    float *pf_PART;         /* split-K partials of the narrow prefill GEMMs: 4 x chunk x hidden */
+    float *pf_PART;         /* split-K partials of the narrow prefill GEMMs: 4 x chunk x hidden, more for a short one */
+    uint64_t pf_part;       /* its floats */
     float *pf_WY;           /* the chunked DeltaNet scan's per-(head, sub-chunk) workspace */
 
     /* the pinned step descriptor's upload: the next write to h_step waits
@@ -512,15 +513,18 @@ sg_err sg_gpu_run_op(sg_gpu *g, const char *kernel, void *a, void *b, void *out,
             sg_failed(e = need(out, (uint64_t)N * M * 4, "Y"))) return e;
         if (sg_failed(e = push(ins, 3))) return e;
         void *t;
-        const uint64_t qb = ((uint64_t)M * K + 255) / 256 * 256, db = ((uint64_t)M * (K / 32) * 2 + 255) / 256 * 256;
-        const uint64_t xb = ((uint64_t)N * K * 4 + 255) / 256 * 256, pc = (uint64_t)4 * N * M;   /* split-K partials */
+        /* few tokens: straight from the blocks; else the two planes and the block-major scales first */
+        const bool raw = N <= sgk_gemm_raw_tokens();
+        const uint64_t qb = raw ? 0 : ((uint64_t)M * K + 255) / 256 * 256, db = raw ? 0 : ((uint64_t)M * (K / 32) * 2 + 255) / 256 * 256;
+        const uint64_t xb = ((uint64_t)N * K * 4 + 255) / 256 * 256, pc = (uint64_t)(raw ? 12 : 4) * N * M;   /* split-K partials */
         if (sg_failed(e = scratch(g, qb + 2 * db + xb + pc * 4, &t))) return e;
         int8_t *qs = t;
         uint16_t *d = (uint16_t *)((char *)t + qb), *dt = (uint16_t *)((char *)t + qb + db);
         uint16_t *xs = (uint16_t *)((char *)t + qb + 2 * db);
         float *part = (float *)((char *)t + qb + 2 * db + xb);
-        hipError_t he = sgk_repack_q8(DEV(b), M, K, qs, d, dt, M, 0, 1, s);
-        if (he == hipSuccess) he = sgk_gemm_q8(DEV(a), qs, dt, DEV(out), N, M, K, xs, part, pc, s);
+        hipError_t he = raw ? hipSuccess : sgk_repack_q8(DEV(b), M, K, qs, d, dt, M, 0, 1, s);
+        if (he == hipSuccess)
+            he = sgk_gemm_q8(DEV(a), raw ? NULL : qs, raw ? NULL : dt, raw ? DEV(b) : NULL, DEV(out), N, M, K, xs, part, pc, s);
         return finish(g, he, outs, 1);
     }
     return errf("gpu: unknown kernel '%s'", kernel);
@@ -1687,12 +1691,16 @@ static sg_err prefill_alloc(sg_gpu *g, uint32_t chunk) {
     if (c->ffn_hidden > kmax) kmax = c->ffn_hidden;
     if (g->attn_width > kmax) kmax = g->attn_width;
     if (g->value_dim > kmax) kmax = g->value_dim;
+    const uint64_t few = n < sgk_gemm_raw_tokens() ? n : sgk_gemm_raw_tokens();   /* a short chunk's products split K up to 12 ways, the wide ones 2 */
+    uint64_t part = (12 * few > 4 * n ? 12 * few : 4 * n) * c->hidden;
+    if (part < 4 * few * c->ffn_hidden) part = 4 * few * c->ffn_hidden;
     uint64_t sizes[] = { n * sizeof(sgk_step), n * c->hidden * 4, n * c->hidden * 4, n * in_rows * 4,
                          n * g->conv_dim * 4 + 4, n * g->value_dim * 4 + 4, n * g->value_dim * 4 + 4,
                          n * g->attn_width * 4 + 4, n * c->ffn_hidden * 4, ah * 4, ah * 4, ah * c->head_dim * 4,
-                         n * kmax * 4, 4 * n * c->hidden * 4, sgk_delta_ws_floats(c->n_v_heads, chunk) * 4 + 4,
+                         n * kmax * 4, part * 4, sgk_delta_ws_floats(c->n_v_heads, chunk) * 4 + 4,
                          n * kmax * 4 };
     sg_err e = SG_OK;
+    g->pf_part = part;
     for (size_t i = 0; i < sizeof bufs / sizeof *bufs && !sg_failed(e); i++) e = dzalloc(g, sizes[i], bufs[i]);
     if (!sg_failed(e) && hipHostMalloc((void **)&g->pf_hsteps, n * sizeof(sgk_step), 0) != hipSuccess)
         e = (sg_err){"gpu: hipHostMalloc failed"};
@@ -1708,8 +1716,8 @@ static sg_err prefill_alloc(sg_gpu *g, uint32_t chunk) {
 static hipError_t gemm_rows_x(sg_gpu *g, const dmat *M, const float *X, uint32_t ldx, float *Y, uint32_t ldy,
                               uint32_t n, int epi, const float *post_nw, int *ready, int xs_ready, uint16_t *xs) {
     sgk_gemm_args a = { X, M->qs, M->dt, M->wf, Y, n, M->rows, M->cols, ldx, ldy, epi, xs, g->pf_PART,
-                        (uint64_t)4 * g->pf_chunk * g->cfg.hidden, NULL, 0.0f, xs_ready, post_nw, g->cfg.rms_eps,
-                        post_nw ? ready : NULL, NULL };
+                        g->pf_part, NULL, 0.0f, xs_ready, post_nw, g->cfg.rms_eps,
+                        post_nw ? ready : NULL, NULL, NULL };
     if (ready) *ready = 0;
     return sgk_gemm(&a, g->stream);
 }
@@ -1731,7 +1739,7 @@ static hipError_t gemm_rows_norm_x(sg_gpu *g, const dmat *M, const float *X, con
         return e != hipSuccess ? e : gemm_rows(g, M, g->pf_Xn, H, Y, ldy, n, epi, NULL, NULL);
     }
     sgk_gemm_args a = { X, M->qs, M->dt, M->wf, Y, n, M->rows, M->cols, H, ldy, epi, xs, g->pf_PART,
-                        (uint64_t)4 * g->pf_chunk * H, nw, g->cfg.rms_eps, xs_ready, NULL, 0.0f, NULL, ys };
+                        g->pf_part, nw, g->cfg.rms_eps, xs_ready, NULL, 0.0f, NULL, ys, NULL };
     return sgk_gemm(&a, g->stream);
 }
 

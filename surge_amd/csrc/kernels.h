@@ -322,10 +322,13 @@ typedef struct {
     uint16_t *ys;            /* SGK_EPI_SWIGLU, Q8 W: the SwiGLU outputs written as the next product's bf16
                               * split (the xs layout, N rows of M/2, (M/2) % 32 == 0) instead of into Y;
                               * must not alias xs */
+    const uint8_t *raw;      /* instead of qs and dt: W as the file's 34-byte blocks (any alignment), for a
+                              * plain store of at most sgk_gemm_raw_tokens() rows */
 } sgk_gemm_args;
 /* Q8 W needs K % 32 == 0, ldx % 4 == 0 and X 16-byte aligned. */
 hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s);
-hipError_t sgk_gemm_q8(const float *X, const int8_t *qs, const uint16_t *dt, float *Y,
+uint32_t sgk_gemm_raw_tokens(void);
+hipError_t sgk_gemm_q8(const float *X, const int8_t *qs, const uint16_t *dt, const uint8_t *raw, float *Y,
                        uint32_t N, uint32_t M, uint32_t K, uint16_t *xs, float *part,
                        uint64_t part_cap, hipStream_t s);
 

@@ -1013,31 +1013,50 @@ extern "C" hipError_t sgk_gemv_raw(const uint8_t *w, uint32_t rows, uint32_t col
 // Q8_0 repack: 34-byte blocks -> int8 plane + f16 scale plane
 // ---------------------------------------------------------------------------
 
-__global__ void k_repack_q8(const uint8_t *src, uint32_t rows, uint32_t cols, int8_t *qs,
-                            uint16_t *d, uint16_t *dt, uint32_t ld, uint32_t row0, uint32_t step) {
-    const uint32_t nbl = cols >> 5;
-    const uint64_t b = (uint64_t)blockIdx.x * TPB + threadIdx.x;
-    if (b >= (uint64_t)rows * nbl) return;
-    const uint32_t r = (uint32_t)(b / nbl), j = (uint32_t)(b % nbl);
-    const uint8_t *p = src + b * 34;
-    const uint64_t dr = (uint64_t)row0 + (uint64_t)r * step;
-    const uint16_t dv = (uint16_t)(p[0] | (p[1] << 8));
-    d[dr * nbl + j] = dv;
-    if (dt) dt[(uint64_t)j * ld + dr] = dv;
-    uint32_t *o = (uint32_t *)(qs + dr * cols + (uint64_t)j * 32);
+// Workgroup: 64 rows x 8 blocks (272 consecutive bytes of a row). Thread: 16
+// weights of one row, loaded where they lie (any alignment) and stored
+// aligned; the scales go through LDS so that the block-major copy is written
+// in runs of rows. Bound by memory, twice the matrix's bytes: 95 MB of blocks
+// in 47 us (125 with byte loads and the copy written one row at a time).
+#define RP_R 64
+#define RP_B 8
+typedef uint32_t v4u_a1 __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint16_t u16_a1 __attribute__((aligned(1)));
+__global__ void __launch_bounds__(TPB) k_repack_q8(const uint8_t *src, uint32_t rows, uint32_t cols, int8_t *qs,
+                                                   uint16_t *d, uint16_t *dt, uint32_t ld, uint32_t row0, uint32_t step) {
+    __shared__ uint16_t sc[RP_B][RP_R];
+    const uint32_t nbl = cols >> 5, t = threadIdx.x, nby = (nbl + RP_B - 1) / RP_B;
+    const uint32_t jb = blockIdx.x % nby * RP_B, r0 = blockIdx.x / nby * RP_R;
+    const uint32_t j = t >> 1 & 7, half = t & 1, blk = jb + j;
 #pragma unroll
-    for (int k = 0; k < 8; k++)
-        o[k] = (uint32_t)p[2 + 4 * k] | ((uint32_t)p[3 + 4 * k] << 8) |
-               ((uint32_t)p[4 + 4 * k] << 16) | ((uint32_t)p[5 + 4 * k] << 24);
+    for (uint32_t u = 0; u < 4; u++) {
+        const uint32_t r = (t >> 4) + 16 * u, row = r0 + r;
+        if (row >= rows || blk >= nbl) continue;
+        const uint8_t *p = src + ((uint64_t)row * nbl + blk) * 34;
+        const uint64_t dr = (uint64_t)row0 + (uint64_t)row * step;
+        const v4u_a1 v = *(const v4u_a1 *)(p + 2 + 16 * half);
+        *(v4u *)(qs + dr * cols + (uint64_t)blk * 32 + 16 * half) = v;
+        if (!half) {
+            const uint16_t dv = *(const u16_a1 *)p;
+            d[dr * nbl + blk] = dv;
+            sc[j][r] = dv;
+        }
+    }
+    if (!dt) return;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = t; i < RP_R * RP_B; i += TPB) {
+        const uint32_t jj = i / RP_R, r = i % RP_R, row = r0 + r;
+        if (row < rows && jb + jj < nbl) dt[(uint64_t)(jb + jj) * ld + row0 + (uint64_t)row * step] = sc[jj][r];
+    }
 }
 
 extern "C" hipError_t sgk_repack_q8(const uint8_t *src, uint32_t rows, uint32_t cols,
                                     int8_t *qs, uint16_t *d, uint16_t *dt, uint32_t ld, uint32_t row0,
                                     uint32_t row_step, hipStream_t s) {
-    const uint64_t n = (uint64_t)rows * (cols >> 5);
+    const uint64_t n = (uint64_t)((rows + RP_R - 1) / RP_R) * (((cols >> 5) + RP_B - 1) / RP_B);
     if (!n) return hipSuccess;
-    hipLaunchKernelGGL(k_repack_q8, dim3((unsigned)((n + TPB - 1) / TPB)), dim3(TPB), 0, s, src,
-                       rows, cols, qs, d, dt, ld, row0, row_step);
+    hipLaunchKernelGGL(k_repack_q8, dim3((unsigned)n), dim3(TPB), 0, s, src, rows, cols, qs, d, dt, ld, row0, row_step);
     return hipGetLastError();
 }
 
@@ -4621,6 +4640,187 @@ k_gemm_q8_wide(const uint16_t *xs, const int8_t *qs, const uint16_t *d, float *Y
             }
 }
 
+// Few-token form (N <= 16 * GF_NT_MAX): a product over a short prompt or a ragged last
+// chunk. Bound by HBM (every weight once), so it is built around the weight
+// stream: a wave owns 32 weight rows and every token, its weights go from
+// memory through the wave's own LDS into MFMA fragments, four Q8_0 blocks at a
+// time (a row's four blocks are one 128-byte line), converted to bf16 in
+// registers, with the next four in flight while these are multiplied. X (the bf16 hi | lo split) goes through LDS,
+// staged for the four waves' 128 rows at a time. K is split over workgroups
+// until about three per CU run, the partials summed in order by the reduces
+// below. Per (block, token tile, weight tile) the arithmetic is gm_tile_step's.
+// RAW: the weights are the file's 34-byte blocks (any alignment).
+// 40 tokens of 5120 x 17408 from blocks: 40 us (repack 124 us and 113 us in
+// the 128-token tile before), 8 tokens 31 us (94 MB at 3 TB/s; the blocks'
+// alignment costs some), 76 tokens 54 us; 34816 x 5120 at 76 tokens 125 (147).
+// Past 80 tokens the LDS for X leaves one workgroup a CU, and the tile
+// of the wide form is used well. Two blocks per X stage from 49 tokens on keep
+// two workgroups a CU (76 tokens: 74 -> 54 us); below that they cost 1-3%.
+#define GF_NT_MAX 5
+#define GF_TM 128
+#define GF_S_MAX 12
+#ifndef GF_XB
+#define GF_XB(NT) ((NT) <= 3 ? 4 : 2)     // blocks per X stage
+#endif
+__device__ __forceinline__ bf16x8 q8_frag(v2u q) {      // 8 int8 -> 8 bf16, exact (as gm_stage_q16)
+    v4u o;
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+        const uint32_t u = q[p >> 1] >> (16 * (p & 1));
+        const float f0 = (float)(int32_t)(int8_t)(u & 0xffu), f1 = (float)(int32_t)(int8_t)((u >> 8) & 0xffu);
+        o[p] = __builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
+    }
+    return __builtin_bit_cast(bf16x8, o);
+}
+struct gf_w {            // four blocks of the wave's 32 rows: 16 weights in each of 4 rows, 2 scales
+    v4u q[4];
+    uint16_t d[2];
+};
+
+template <int EPI, int NT, bool RAW>
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_gemm_q8_few(const uint16_t *xs, const void *w, const uint16_t *d, float *Y, uint32_t N, uint32_t M, uint32_t K,
+              uint32_t ldy, uint64_t ysplit) {
+    constexpr int XB = GF_XB(NT);
+    __shared__ __align__(16) uint8_t xt[2][XB][NT * 16 * 128];     // [buffer][block][token][hi 64 B | lo 64 B, swizzled]
+    __shared__ __align__(16) uint8_t wt[TPB / 64][32 * 128];       // [wave][row][4 blocks of 32 int8, swizzled]
+    __shared__ float ws[TPB / 64][4][32];                          // [wave][block][row]
+    constexpr int XR = NT * XB / 2;                                 // 16-byte chunks of a stage per thread
+    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 15, lg = lane >> 4;
+    const uint32_t nblk = K >> 5, m0 = blockIdx.x * GF_TM + wave * 32;
+    const uint32_t kb0 = (uint32_t)((uint64_t)nblk * blockIdx.y / gridDim.y);
+    const uint32_t kb1 = (uint32_t)((uint64_t)nblk * (blockIdx.y + 1) / gridDim.y), kl = kb1 - 1;
+    // the wave's weights: lane loads half block lane % 8 of row lane / 8 (+ 8, 16,
+    // 24), so four neighbouring lanes share a line (a fragment's own order, 16
+    // rows in 16 neighbouring lanes, loads a line per lane: 60 us where this
+    // takes 25), and puts them into the wave's own LDS, read back as fragments
+    const uint32_t r8 = lane >> 3, ch = lane & 7;
+    const size_t rb = RAW ? (size_t)nblk * 34 : (size_t)K;
+    const uint8_t *wp[4], *dp[2];
+#pragma unroll
+    for (int i = 0; i < 4; i++) wp[i] = (const uint8_t *)w + min(m0 + i * 8 + r8, M - 1) * rb + (ch & 1) * 16 + (RAW ? 2 : 0);
+#pragma unroll
+    for (int i = 0; i < 2; i++)        // scale i*64 + lane: RAW row / 4, block % 4; else block / 32, row % 32
+        dp[i] = RAW ? (const uint8_t *)w + min(m0 + i * 16 + (lane >> 2), M - 1) * rb
+                    : (const uint8_t *)(d + min(m0 + (lane & 31), M - 1));
+    auto load_w = [&](gf_w &b, uint32_t s) {
+        const uint32_t blk = min(s + (ch >> 1), kl);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            b.q[i] = RAW ? (v4u) * (const v4u_a1 *)(wp[i] + (size_t)blk * 34) : *(const v4u *)(wp[i] + (size_t)blk * 32);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            b.d[i] = RAW ? *(const u16_a1 *)(dp[i] + (size_t)min(s + (lane & 3), kl) * 34)
+                         : ((const uint16_t *)dp[i])[(size_t)min(s + 2 * i + (lane >> 5), kl) * M];
+    };
+    auto store_w = [&](const gf_w &b) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) *(v4u *)&wt[wave][(i * 8 + r8) * 128 + ((ch ^ r8) << 4)] = b.q[i];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            if (RAW) ws[wave][lane & 3][i * 16 + (lane >> 2)] = h2f(b.d[i]);
+            else ws[wave][2 * i + (lane >> 5)][lane & 31] = h2f(b.d[i]);
+        }
+    };
+    // X staging: thread t takes chunks t, t + 256, ... of the stage's
+    // [XB blocks][NT * 16 tokens][8 chunks] (tokens past N repeat the last)
+    v4u xr[XR];
+    auto load_x = [&](uint32_t s) {
+#pragma unroll
+        for (int u = 0; u < XR; u++) {
+            const uint32_t i = t + u * TPB, j = i / (NT * 128), n = i / 8 % (NT * 16), c = i & 7;
+            xr[u] = *(const v4u *)(xs + ((size_t)min(s + j, kl) * N + min(n, N - 1)) * 64 + c * 8);
+        }
+    };
+    auto store_x = [&](uint32_t buf) {
+#pragma unroll
+        for (int u = 0; u < XR; u++) {
+            const uint32_t i = t + u * TPB, j = i / (NT * 128), n = i / 8 % (NT * 16), c = i & 7;
+            *(v4u *)&xt[buf][j][n * 128 + ((c ^ (n & 7)) << 4)] = xr[u];
+        }
+    };
+    f32x4 acc[NT][2];
+#pragma unroll
+    for (int a = 0; a < NT; a++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) acc[a][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const uint32_t xo = li * 128 + ((lg ^ (li & 7)) << 4);
+    const uint32_t wo = li * 128 + (((lg >> 1) ^ (li & 7)) << 4) + (lg & 1) * 8;
+    auto multiply = [&](int o, uint32_t s, uint32_t buf) {         // blocks o .. o + XB - 1 of the four at s
+#pragma unroll
+        for (int j = o; j < o + XB; j++) {
+            if (s + j >= kb1) break;
+            const bf16x8 b0 = q8_frag(*(const v2u *)&wt[wave][wo ^ (j * 32)]), b1 = q8_frag(*(const v2u *)&wt[wave][2048 + (wo ^ (j * 32))]);
+            const float d0 = ws[wave][j][li], d1 = ws[wave][j][16 + li];
+#pragma unroll
+            for (int a = 0; a < NT; a++) {
+                const bf16x8 ah = *(const bf16x8 *)&xt[buf][j - o][a * 2048 + xo], al = *(const bf16x8 *)&xt[buf][j - o][a * 2048 + (xo ^ 64)];
+                const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+                f32x4 p0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, b0, z, 0, 0, 0);
+                f32x4 p1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, b1, z, 0, 0, 0);
+                p0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, b0, p0, 0, 0, 0);
+                p1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, b1, p1, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    acc[a][0][e] = fmaf(d0, p0[e], acc[a][0][e]);
+                    acc[a][1][e] = fmaf(d1, p1[e], acc[a][1][e]);
+                }
+            }
+        }
+    };
+    gf_w wv;
+    load_x(kb0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(wv, kb0);
+    store_x(0);
+    __syncthreads();
+    uint32_t buf = 0;
+    for (uint32_t s = kb0; s < kb1; s += 4) {
+        store_w(wv);                            // (this wave's LDS operations run in order)
+#pragma unroll
+        for (int o = 0; o < 4; o += XB, buf ^= 1) {
+            load_x(min(s + o + XB, kl));
+            __builtin_amdgcn_sched_barrier(0);
+            if (o == 0) load_w(wv, min(s + 4, kl));
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(o, s, buf);
+            store_x(buf ^ 1);
+            __syncthreads();
+        }
+    }
+    // lane holds D[i = 4*lg + e (token)][j = li (row)] of each tile
+    Y += (size_t)blockIdx.y * ysplit;
+#pragma unroll
+    for (int a = 0; a < NT; a++)
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t n = a * 16 + lg * 4 + e, m = m0 + c * 16 + li;
+                const float v = acc[a][c][e];
+                if (EPI == SGK_EPI_SWIGLU || EPI == SGK_EPI_SWIGLU_XS) {
+                    const float up = lane_xor1(v);            // column m+1 lives in lane li^1
+                    if (!(li & 1) && n < N && m + 1 < M) {
+                        if (EPI == SGK_EPI_SWIGLU) Y[(size_t)n * ldy + (m >> 1)] = silu(v) * up;
+                        else xs_put((uint16_t *)Y, N, n, m >> 1, silu(v) * up);
+                    }
+                } else if (n < N && m < M) {
+                    if (EPI == SGK_EPI_ADD) Y[(size_t)n * ldy + m] += v;
+                    else Y[(size_t)n * ldy + m] = v;
+                }
+            }
+}
+
+template <int EPI, bool RAW>
+static hipError_t few_launch(const sgk_gemm_args *a, float *Y, uint32_t ldy, uint64_t ysplit, uint32_t S, hipStream_t s) {
+    const dim3 grid((a->M + GF_TM - 1) / GF_TM, S);
+    const void *w = RAW ? (const void *)a->raw : (const void *)a->qs;
+#define FEW(T) case T: hipLaunchKernelGGL((k_gemm_q8_few<EPI, T, RAW>), grid, dim3(TPB), 0, s, a->xs, w, a->dt, Y, a->N, a->M, a->K, ldy, ysplit); break
+    switch ((a->N + 15) / 16) { FEW(1); FEW(2); FEW(3); FEW(4); FEW(5); default: return hipErrorInvalidValue; }
+#undef FEW
+    return hipGetLastError();
+}
+
 // Split-K epilogue: the S partials P[s][N][M] summed in order, then the GEMM
 // epilogue (store, += residual, SwiGLU on (gate, up) column pairs).
 template <int EPI>
@@ -4767,6 +4967,29 @@ __global__ void __launch_bounds__(TPB) k_gemm_f32(const float *X, const float *W
     }
 }
 
+// The epilogue of a product whose S partials are in a->part.
+static hipError_t splitk_finish(const sgk_gemm_args *a, uint32_t S, int epi, float *Yo, hipStream_t s) {
+    if (a->epi == SGK_EPI_ADD && a->post_nw && a->post_done && a->ldy % 4 == 0 && a->M % 32 == 0 &&
+        !((uintptr_t)a->Y & 15) && !((uintptr_t)a->post_nw & 15)) {
+        // the residual add fused with the next product's RMSNorm and split (into this
+        // product's xs, which it has finished reading)
+        auto red = S == 2 ? k_splitk_reduce_rms<2> : S == 3 ? k_splitk_reduce_rms<3> : S == 4 ? k_splitk_reduce_rms<4> :
+                   S == 6 ? k_splitk_reduce_rms<6> : S == 8 ? k_splitk_reduce_rms<8> : k_splitk_reduce_rms<GF_S_MAX>;
+        hipLaunchKernelGGL(red, dim3(a->N), dim3(TPB), 0, s, a->part, a->N, a->M, a->Y, a->ldy, a->post_nw, a->post_eps,
+                           a->xs);
+        *a->post_done = 1;
+        return hipGetLastError();
+    }
+    const uint32_t rg = (uint32_t)min(((uint64_t)a->N * a->M + TPB - 1) / TPB, (uint64_t)4096);
+#define GR(E) hipLaunchKernelGGL((k_splitk_reduce<E>), dim3(rg), dim3(TPB), 0, s, a->part, S, a->N, a->M, Yo, a->ldy)
+    if (epi == SGK_EPI_ADD) GR(SGK_EPI_ADD);
+    else if (epi == SGK_EPI_SWIGLU) GR(SGK_EPI_SWIGLU);
+    else if (epi == SGK_EPI_SWIGLU_XS) GR(SGK_EPI_SWIGLU_XS);
+    else GR(SGK_EPI_STORE);
+#undef GR
+    return hipGetLastError();
+}
+
 extern "C" hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s) {
     if (!a->N || !a->M || !a->K) return hipSuccess;
     if (a->epi == SGK_EPI_SWIGLU && (a->M & 1)) return hipErrorInvalidValue;
@@ -4775,8 +4998,8 @@ extern "C" hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s) {
     const int epi = a->ys ? SGK_EPI_SWIGLU_XS : a->epi;
     float *const Yo = a->ys ? (float *)a->ys : a->Y;
     if (a->nw && !a->qs) return hipErrorInvalidValue;      // the fused RMSNorm is part of the Q8 split
-    if (a->qs) {
-        if (a->K % 32 || !a->xs || !a->dt || a->ldx % 4 || ((uintptr_t)a->X & 15) || ((uintptr_t)a->xs & 15))
+    if (a->qs || a->raw) {
+        if (a->K % 32 || !a->xs || (!a->dt && !a->raw) || a->ldx % 4 || ((uintptr_t)a->X & 15) || ((uintptr_t)a->xs & 15))
             return hipErrorInvalidValue;
         const uint32_t k4 = a->K / 4;
         const uint64_t total = (uint64_t)a->N * k4;
@@ -4791,6 +5014,27 @@ extern "C" hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s) {
             hipLaunchKernelGGL(k_split_bf16, dim3(sg), dim3(TPB), 0, s, a->X, a->ldx, a->N, a->K, a->xs);
         }
         const int kind = gemm_kind();
+        if (a->N <= 16 * GF_NT_MAX && (kind == GEMM_WIDE || a->raw)) {
+            // three workgroups per CU, at least 16 blocks of K each, partials that fit (the
+            // fused reduce is built for these counts): the 5120 x 17408 product of 40 tokens
+            // took 52 us in 8 splits, 40 in 12, 46 in 16
+            const uint32_t mt = (a->M + GF_TM - 1) / GF_TM, nbl = a->K / 32, per = max(1u, 3 * (uint32_t)device_cus() / mt);
+            uint32_t S = 1;
+            for (uint32_t v : {2u, 3u, 4u, 6u, 8u, (uint32_t)GF_S_MAX})
+                if (a->part && v <= per && nbl / v >= 16 && (uint64_t)v * a->N * a->M <= a->part_cap) S = v;
+            if (S > 1) {
+                const uint64_t ys = (uint64_t)a->N * a->M;
+                hipError_t e = a->raw ? few_launch<SGK_EPI_STORE, true>(a, a->part, a->M, ys, S, s)
+                                      : few_launch<SGK_EPI_STORE, false>(a, a->part, a->M, ys, S, s);
+                return e != hipSuccess ? e : splitk_finish(a, S, epi, Yo, s);
+            }
+            if (a->raw) return epi == SGK_EPI_STORE ? few_launch<SGK_EPI_STORE, true>(a, a->Y, a->ldy, 0, 1, s) : hipErrorInvalidValue;
+            if (epi == SGK_EPI_ADD) return few_launch<SGK_EPI_ADD, false>(a, a->Y, a->ldy, 0, 1, s);
+            if (epi == SGK_EPI_SWIGLU) return few_launch<SGK_EPI_SWIGLU, false>(a, a->Y, a->ldy, 0, 1, s);
+            if (epi == SGK_EPI_SWIGLU_XS) return few_launch<SGK_EPI_SWIGLU_XS, false>(a, Yo, a->ldy, 0, 1, s);
+            return few_launch<SGK_EPI_STORE, false>(a, a->Y, a->ldy, 0, 1, s);
+        }
+        if (a->raw) return hipErrorInvalidValue;
         const uint32_t TM = kind == GEMM_WIDE ? GX_TM : GM_TM;
         const uint32_t mb = (a->M + TM - 1) / TM, nb = (a->N + GM_TN - 1) / GM_TN;
         const uint32_t grid = 8 * gm_per_xcd(mb, nb), nblk = a->K / 32, tiles = mb * nb;
@@ -4822,24 +5066,7 @@ extern "C" hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s) {
         }
         if (S > 1) {
             GL(SGK_EPI_STORE, dim3(grid, S), a->part, a->M, (uint64_t)a->N * a->M, 0u);
-            if (a->epi == SGK_EPI_ADD && a->post_nw && a->post_done && a->ldy % 4 == 0 && a->M % 32 == 0 &&
-                !((uintptr_t)a->Y & 15) && !((uintptr_t)a->post_nw & 15)) {
-                // the residual add fused with the next product's RMSNorm and split (into this
-                // product's xs, which it has finished reading)
-                auto red = S == 2 ? k_splitk_reduce_rms<2> : S == 3 ? k_splitk_reduce_rms<3> : k_splitk_reduce_rms<4>;
-                hipLaunchKernelGGL(red, dim3(a->N), dim3(TPB), 0, s, a->part, a->N, a->M, a->Y, a->ldy,
-                                   a->post_nw, a->post_eps, a->xs);
-                *a->post_done = 1;
-                return hipGetLastError();
-            }
-            const uint32_t rg = (uint32_t)min(((uint64_t)a->N * a->M + TPB - 1) / TPB, (uint64_t)4096);
-#define GR(E) hipLaunchKernelGGL((k_splitk_reduce<E>), dim3(rg), dim3(TPB), 0, s, a->part, S, a->N, a->M, Yo, a->ldy)
-            if (epi == SGK_EPI_ADD) GR(SGK_EPI_ADD);
-            else if (epi == SGK_EPI_SWIGLU) GR(SGK_EPI_SWIGLU);
-            else if (epi == SGK_EPI_SWIGLU_XS) GR(SGK_EPI_SWIGLU_XS);
-            else GR(SGK_EPI_STORE);
-#undef GR
-            return hipGetLastError();
+            return splitk_finish(a, S, epi, Yo, s);
         }
         uint32_t full = grid, S2 = 1;
         if (a->part && grid > slots) {
@@ -4877,12 +5104,14 @@ extern "C" hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s) {
     return hipGetLastError();
 }
 
-extern "C" hipError_t sgk_gemm_q8(const float *X, const int8_t *qs, const uint16_t *dt, float *Y,
+extern "C" hipError_t sgk_gemm_q8(const float *X, const int8_t *qs, const uint16_t *dt, const uint8_t *raw, float *Y,
                                   uint32_t N, uint32_t M, uint32_t K, uint16_t *xs, float *part,
                                   uint64_t part_cap, hipStream_t s) {
     sgk_gemm_args a = {X, qs, dt, NULL, Y, N, M, K, K, M, SGK_EPI_STORE, xs, part, part_cap};
+    a.raw = raw;
     return sgk_gemm(&a, s);
 }
+extern "C" uint32_t sgk_gemm_raw_tokens(void) { return 16 * GF_NT_MAX; }
 
 // ---------------------------------------------------------------------------
 // Measurement kernels: a plain streaming read (16-byte non-temporal loads, a

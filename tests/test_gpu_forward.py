@@ -465,6 +465,25 @@ def test_prefill_gemm_round_split_matches_serial(gpu, monkeypatch, kind, slots):
     syn.close()
 
 
+@pytest.mark.parametrize("n", [1, 40, 80])
+def test_short_prefill_matches_serial(gpu, n):
+    """The few-token products with every epilogue: a plain store, the residual
+    add alone (K too short to split) and behind a split K with the next norm
+    (the down projection, 6144 wide, 12 ways), SwiGLU into the next split. A
+    prompt in one short chunk against the serial forward (2e-4, same argmax)."""
+    syn = S.Synth(dict(WIDE, ffn_hidden=6144), S.SG_T_Q8_0, seed=27)
+    gpu.load_model(syn.model)
+    gpu.state_new(96)
+    prompt = np.random.default_rng(n).integers(0, WIDE["vocab"], n).tolist()
+    serial = None
+    for p, t in enumerate(prompt):
+        serial = gpu.forward(t, p)
+    last = gpu.prefill(prompt, chunk=128)
+    assert rel(last, serial) < 2e-4
+    assert int(np.argmax(last)) == int(np.argmax(serial))
+    syn.close()
+
+
 @pytest.mark.parametrize("slots", [None, "12"])
 def test_prefill_gemm_warp_specialised_matches_plain(gpu, monkeypatch, slots):
     """The three prefill GEMM forms run the same per-step arithmetic (two

@@ -680,6 +680,22 @@ def test_matmul_q8_prefill_gemm(gpu, N, M, K):
     assert_close(yb.array.reshape(N, M), want)
 
 
+@pytest.mark.parametrize("N,M,K", [(2, 5, 32), (16, 127, 160), (17, 129, 96), (33, 260, 1120), (48, 31, 6144),
+                                   (49, 128, 2080), (64, 385, 64), (80, 257, 544), (81, 130, 288)])
+def test_matmul_q8_few_tokens(gpu, N, M, K):
+    """The few-token product at the edges of its token tiles, of its 128-row
+    tiles and of its four-block stages (K / 32 from 1 to 192, split over K
+    where that is at least 16 blocks each, up to 12 ways), and the first count
+    past it; the split of x holds to 2^-17 a term, so 1e-4 of the largest value."""
+    rng = np.random.default_rng(N + M + K)
+    X = rng.standard_normal(N * K).astype(np.float32)
+    raw = q8_matrix(rng, M, K, sigma=1.0)
+    xb, wb, yb = gpu.buf(X), gpu.buf(raw), gpu.buf(np.zeros(N * M, np.float32))
+    gpu.run_op("k_matmul_q8", xb, wb, yb, [N, M, K])
+    want = np.stack([oracle_matvec_q8(raw, np.ascontiguousarray(X[n * K:(n + 1) * K]), M, K) for n in range(N)])
+    assert_close(yb.array.reshape(N, M), want, 1e-4)
+
+
 @pytest.mark.parametrize("kind,slots", [("wide", "14"), ("ws", "28")])
 def test_matmul_q8_prefill_gemm_round_split(gpu, monkeypatch, kind, slots):
     """The prefill GEMM's round split on a 256 x 2048 x 1792 product: the wide
