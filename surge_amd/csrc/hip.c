@@ -921,7 +921,9 @@ sg_err sg_gpu_run_attn_prefill(sg_gpu *g, void *q, void *k, void *v, void *out, 
     uint64_t kvb = (uint64_t)(base + n) * nkv * hd * 2;
     if (sg_failed(e = need(q, (uint64_t)n * nh * qs * 4, "q")) || sg_failed(e = need(k, kvb, "k")) ||
         sg_failed(e = need(v, kvb, "v")) || sg_failed(e = need(out, (uint64_t)n * nh * hd * 4, "out"))) return e;
-    uint64_t ah = (uint64_t)n * nh * SGK_PREFILL_SPLITS;
+    const bool flash = (hd == 64 || hd == 128 || hd == 256) && qs % 4 == 0;
+    const uint32_t ms = flash ? sgk_flash_max_splits(n) : SGK_PREFILL_SPLITS;
+    uint64_t ah = (uint64_t)n * nh * ms;
     uint64_t steps_b = ((uint64_t)n * sizeof(sgk_step) + 255) / 256 * 256;
     void *t;
     if (sg_failed(e = scratch(g, steps_b + ah * (2 + hd) * 4, &t))) return e;
@@ -937,12 +939,12 @@ sg_err sg_gpu_run_attn_prefill(sg_gpu *g, void *q, void *k, void *v, void *out, 
     sgk_attn A = {0};
     A.q = DEV(q); A.kc = DEV(k); A.vc = DEV(v); A.m = mm; A.s = ss; A.acc = aa; A.out = DEV(out); A.steps = t;
     A.n_heads = nh; A.n_kv = nkv; A.hd = hd; A.q_stride = qs; A.q_tok = nh * qs; A.out_tok = nh * hd;
-    A.max_splits = SGK_PREFILL_SPLITS; A.ntok = n; A.scale = fbits(p[6]); A.prefill = 1;
+    A.max_splits = ms; A.ntok = n; A.scale = fbits(p[6]); A.prefill = 1;
     A.seq = base + n;
     /* The prefill path's kernel: the MFMA flash pass (deep chunks split over
      * keys and merged by the combine) for head_dim 64/128/256 with float4 q
      * rows; the split-K kernels per token otherwise. */
-    if ((hd == 64 || hd == 128 || hd == 256) && qs % 4 == 0) {
+    if (flash) {
         he = sgk_attn_flash(&A, g->stream);
     } else {
         he = sgk_attn_partial(&A, g->stream);
@@ -984,7 +986,7 @@ sg_err sg_gpu_run_attn_chunk(sg_gpu *g, void *in, void *w, void *kv, void *out, 
     /* scratch: step descriptors, the chunk's RoPE rows, the normed and roped q
      * (the caller's rows stay as they are) and the key splits' partials */
     const uint64_t steps_b = ((uint64_t)n * sizeof(sgk_step) + 255) / 256 * 256, cs_b = ((uint64_t)n * rd * 4 + 255) / 256 * 256;
-    const uint64_t q_f = (uint64_t)n * nh * hd, ah = (uint64_t)n * nh * SGK_PREFILL_SPLITS;
+    const uint64_t q_f = (uint64_t)n * nh * hd, ah = (uint64_t)n * nh * sgk_flash_max_splits(n);
     void *t;
     if (sg_failed(e = scratch(g, steps_b + cs_b + (q_f + ah * (2 + hd)) * 4, &t))) return e;
     hipStream_t s = g->stream;
@@ -999,7 +1001,7 @@ sg_err sg_gpu_run_attn_chunk(sg_gpu *g, void *in, void *w, void *kv, void *out, 
     A.src = rows; A.src_tok = (uint32_t)row; A.src_stride = 2 * hd;
     A.gate = rows + hd; A.gate_tok = (uint32_t)row; A.gate_stride = 2 * hd;
     A.steps = t; A.n_heads = nh; A.n_kv = nkv; A.hd = hd; A.rope_dim = rd;
-    A.q_stride = hd; A.q_tok = nh * hd; A.out_tok = nh * hd; A.max_splits = SGK_PREFILL_SPLITS;
+    A.q_stride = hd; A.q_tok = nh * hd; A.out_tok = nh * hd; A.max_splits = sgk_flash_max_splits(n);
     A.ntok = n; A.seq = (uint32_t)cap; A.scale = (float)(1.0 / sqrt((double)hd)); A.prefill = 1;
     hipError_t he = sgk_rope_rows(inv, rd, base, n, cs, t, s);
     if (he == hipSuccess) he = sgk_attn_prep(&A, wn, wn + hd, cs, base, fbits(p[7]), s);
@@ -1686,7 +1688,9 @@ static sg_err prefill_alloc(sg_gpu *g, uint32_t chunk) {
     const sg_cfg *c = &g->cfg;
     uint32_t in_rows = 0;
     for (uint32_t i = 0; i < c->n_layers; i++) if (g->ls[i].in.rows > in_rows) in_rows = g->ls[i].in.rows;
-    uint64_t n = chunk, ah = n * c->n_heads * SGK_PREFILL_SPLITS;
+    uint64_t n = chunk, ah = n * SGK_PREFILL_SPLITS;
+    const uint64_t sh = (chunk < SGK_SHORT_CHUNK ? n : SGK_SHORT_CHUNK) * SGK_SHORT_SPLITS;   /* a short (last) chunk splits its keys more ways */
+    ah = (ah > sh ? ah : sh) * c->n_heads;
     uint64_t kmax = c->hidden;                      /* widest GEMM input row */
     if (c->ffn_hidden > kmax) kmax = c->ffn_hidden;
     if (g->attn_width > kmax) kmax = g->attn_width;
@@ -1810,7 +1814,8 @@ static hipError_t prefill_chunk(sg_gpu *g, uint32_t base, uint32_t n) {
             A.q = g->pf_IN; A.kc = L->kc; A.vc = L->vc; A.m = g->pf_m; A.s = g->pf_s; A.acc = g->pf_acc;
             A.out = g->pf_CTX; A.gate = c->attn_output_gate ? g->pf_IN + hd : NULL; A.steps = g->pf_steps;
             A.n_heads = c->n_heads; A.n_kv = c->n_kv_heads; A.hd = hd; A.rope_dim = c->rope_dim; A.q_stride = qs;
-            A.q_tok = in_rows; A.out_tok = g->attn_width; A.max_splits = SGK_PREFILL_SPLITS; A.ntok = n;
+            A.q_tok = in_rows; A.out_tok = g->attn_width; A.ntok = n;
+            A.max_splits = hd == 64 || hd == 128 || hd == 256 ? sgk_flash_max_splits(n) : SGK_PREFILL_SPLITS;
             A.seq = base + n;       /* keys of the chunk's last token: the flash pass splits deep chunks */
             A.scale = (float)(1.0 / sqrt((double)hd)); A.prefill = 1;
             A.kv_ps = hd; A.kv_hs = (uint64_t)g->max_ctx * hd;

@@ -126,6 +126,11 @@ hipError_t sgk_softmax(const float *x, float *out, uint32_t n, hipStream_t s);
  * z*n_heads*max_splits (x hd for acc); its output at out + z*out_tok.
  * Without steps (one-shot per-op calls) seq/n_splits are taken from here. */
 #define SGK_PREFILL_SPLITS 8u
+/* ... and up to this many key splits of the flash pass for a chunk of at most
+ * SGK_SHORT_CHUNK tokens: the split partials a chunk of n tokens may need. */
+#define SGK_SHORT_CHUNK 128u
+#define SGK_SHORT_SPLITS 32u
+static inline uint32_t sgk_flash_max_splits(uint32_t n) { return n <= SGK_SHORT_CHUNK ? SGK_SHORT_SPLITS : SGK_PREFILL_SPLITS; }
 typedef struct {
     float *q;                   /* prep: the fused q|k|v GEMM rows (q normed+roped in place) */
     uint16_t *kc, *vc;          /* f16 caches (layout: kv_ps, kv_hs below) */

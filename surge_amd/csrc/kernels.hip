@@ -2499,7 +2499,21 @@ extern "C" hipError_t sgk_attn_combine(const sgk_attn *a, hipStream_t s);
 // split), when a->m, s, acc hold ntok x n_heads x max_splits partials. The
 // splits write partials and k_attn_combine merges them in split order and
 // applies the gate.
+// A short chunk has fewer pairs still (24 for 76 tokens x 24 heads), and its
+// launch is as long as one workgroup's chain of tiles: while it leaves three
+// quarters of the CUs idle it is split until the chip is full, down to two
+// tiles (128 keys) each. Its partials are few then, so the combine stays short;
+// at 96 pairs (a 512-token chunk) the combine's 25 MB cost what the split saved.
+// 77 tokens of 8 heads at 1024 keys, whole layer call: 54.6 us in 3 splits, 45.5 in 8.
 #define FA_SPLIT_KEYS 512u
+static uint32_t flash_splits(const sgk_attn *a, uint32_t hw) {
+    if (!a->m || !a->s || !a->acc || a->max_splits < 2) return 1;
+    uint32_t S = a->seq > FA_SPLIT_KEYS ? (a->seq + FA_SPLIT_KEYS - 1) / FA_SPLIT_KEYS : 1;
+    S = min(S, min(a->max_splits, SGK_PREFILL_SPLITS));
+    const uint32_t wgs = a->n_heads / hw * ((a->ntok + FA_TQ - 1) / FA_TQ), cus = (uint32_t)device_cus();
+    if (4 * wgs <= cus) S = max(S, min(min(a->seq / (2 * FA_TK), cus / wgs), a->max_splits));
+    return S;
+}
 extern "C" hipError_t sgk_attn_flash(const sgk_attn *a, hipStream_t s) {
     if (!a->ntok || !a->n_heads) return hipSuccess;
     if (!a->steps || !a->n_kv || a->n_heads % a->n_kv || ((uintptr_t)a->q & 15) || a->q_stride % 4 || a->q_tok % 4)
@@ -2507,13 +2521,11 @@ extern "C" hipError_t sgk_attn_flash(const sgk_attn *a, hipStream_t s) {
     if (a->hd != 64 && a->hd != 128 && a->hd != 256) return hipErrorInvalidValue;
     // the output rows (and the split partials) are stored as float4s
     if (((uintptr_t)a->out & 15) || a->out_tok % 4 || (a->acc && ((uintptr_t)a->acc & 15))) return hipErrorInvalidValue;
-    uint32_t S = 1;
-    if (a->m && a->s && a->acc && a->max_splits > 1 && a->seq > FA_SPLIT_KEYS)
-        S = min(a->max_splits, (a->seq + FA_SPLIT_KEYS - 1) / FA_SPLIT_KEYS);
-    sgk_attn k = kv_resolved(a);
-    k.max_splits = S;
     // two query heads per workgroup when their group size allows
     const uint32_t hw = (a->n_heads / a->n_kv) % 2 == 0 ? 2 : 1;
+    const uint32_t S = flash_splits(a, hw);
+    sgk_attn k = kv_resolved(a);
+    k.max_splits = S;
     dim3 grid(a->n_heads / hw, (a->ntok + FA_TQ - 1) / FA_TQ, S);
 #define FLC(H) do { if (hw == 2) hipLaunchKernelGGL((k_attn_flash<H, 2>), grid, dim3(2 * TPB), 0, s, k);       \
                      else hipLaunchKernelGGL((k_attn_flash<H, 1>), grid, dim3(TPB), 0, s, k); } while (0)

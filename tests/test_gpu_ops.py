@@ -944,6 +944,14 @@ def test_attn_prefill_chunk_vs_oracle(gpu, nh, nkv, hd, rd, base, n):
     assert (np.abs(got_kv[0, base:].astype(np.float32) - Ko[base:]) <= ulp).all()
 
 
+@pytest.mark.parametrize("nh,nkv,hd,rd,base,n", [(8, 2, 256, 64, 1024, 77), (2, 1, 128, 32, 4200, 3), (4, 4, 64, 64, 255, 1),
+                                                 (24, 4, 256, 64, 900, 128), (24, 4, 256, 64, 900, 129)])
+def test_attn_chunk_short_splits(gpu, nh, nkv, hd, rd, base, n):
+    """A short chunk split over keys until the chip is full: 8 ways, the most (32),
+    too few keys for two ranges, and both sides of the length that may."""
+    test_attn_prefill_chunk_vs_oracle(gpu, nh, nkv, hd, rd, base, n)
+
+
 @pytest.mark.parametrize("rd,base,n", [(2, 0, 1), (256, 70000, 3), (62, 131, 9)])
 def test_attn_chunk_rope_rows(gpu, rd, base, n):
     """The chunk's RoPE rows (k_rope_rows): one frequency, as many as fit, and a
