@@ -513,10 +513,9 @@ sg_err sg_gpu_run_op(sg_gpu *g, const char *kernel, void *a, void *b, void *out,
             sg_failed(e = need(out, (uint64_t)N * M * 4, "Y"))) return e;
         if (sg_failed(e = push(ins, 3))) return e;
         void *t;
-        /* few tokens: straight from the blocks; else the two planes and the block-major scales first */
-        const bool raw = N <= sgk_gemm_raw_tokens();
+        const bool raw = sgk_gemm_takes_raw(N);         /* else through the repacked planes */
         const uint64_t qb = raw ? 0 : ((uint64_t)M * K + 255) / 256 * 256, db = raw ? 0 : ((uint64_t)M * (K / 32) * 2 + 255) / 256 * 256;
-        const uint64_t xb = ((uint64_t)N * K * 4 + 255) / 256 * 256, pc = (uint64_t)(raw ? 12 : 4) * N * M;   /* split-K partials */
+        const uint64_t xb = ((uint64_t)N * K * 4 + 255) / 256 * 256, pc = (uint64_t)(N <= sgk_gemm_few_tokens() ? 12 : 4) * N * M;   /* split-K partials */
         if (sg_failed(e = scratch(g, qb + 2 * db + xb + pc * 4, &t))) return e;
         int8_t *qs = t;
         uint16_t *d = (uint16_t *)((char *)t + qb), *dt = (uint16_t *)((char *)t + qb + db);
@@ -1695,7 +1694,7 @@ static sg_err prefill_alloc(sg_gpu *g, uint32_t chunk) {
     if (c->ffn_hidden > kmax) kmax = c->ffn_hidden;
     if (g->attn_width > kmax) kmax = g->attn_width;
     if (g->value_dim > kmax) kmax = g->value_dim;
-    const uint64_t few = n < sgk_gemm_raw_tokens() ? n : sgk_gemm_raw_tokens();   /* a short chunk's products split K up to 12 ways, the wide ones 2 */
+    const uint64_t few = n < sgk_gemm_few_tokens() ? n : sgk_gemm_few_tokens();   /* a short chunk's products split K up to 12 ways, the wide ones 2 */
     uint64_t part = (12 * few > 4 * n ? 12 * few : 4 * n) * c->hidden;
     if (part < 4 * few * c->ffn_hidden) part = 4 * few * c->ffn_hidden;
     uint64_t sizes[] = { n * sizeof(sgk_step), n * c->hidden * 4, n * c->hidden * 4, n * in_rows * 4,

@@ -328,11 +328,15 @@ typedef struct {
                               * split (the xs layout, N rows of M/2, (M/2) % 32 == 0) instead of into Y;
                               * must not alias xs */
     const uint8_t *raw;      /* instead of qs and dt: W as the file's 34-byte blocks (any alignment), for a
-                              * plain store of at most sgk_gemm_raw_tokens() rows */
+                              * plain store; see sgk_gemm_takes_raw */
 } sgk_gemm_args;
 /* Q8 W needs K % 32 == 0, ldx % 4 == 0 and X 16-byte aligned. */
 hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s);
-uint32_t sgk_gemm_raw_tokens(void);
+/* Rows X may have for the few-token form; whether N rows are best multiplied by
+ * the file's blocks as they are (with the default form; those that
+ * SURGE_GEMM_* select take the planes only). */
+uint32_t sgk_gemm_few_tokens(void);
+int sgk_gemm_takes_raw(uint32_t N);
 hipError_t sgk_gemm_q8(const float *X, const int8_t *qs, const uint16_t *dt, const uint8_t *raw, float *Y,
                        uint32_t N, uint32_t M, uint32_t K, uint16_t *xs, float *part,
                        uint64_t part_cap, hipStream_t s);

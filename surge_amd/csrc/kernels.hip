@@ -4489,6 +4489,13 @@ struct gx_set {
     v4u x[4];        // X hi and lo of the thread's chunk in its two token rows
     uint32_t d;      // the block scale of the thread's row
 };
+// RAW: the weights are the file's 34-byte blocks; dcol is the row's first scale
+// and dm the 17 half words to the next, wrow the row's bytes. Unaligned rows
+// and a scale per line cost the product some 28 us per 512 tokens of 17408 x
+// 5120 where a repack costs 47 (the call: 247 -> 228 us), so a caller's blocks
+// are multiplied as they are up to GX_RAW_TOKENS and repacked past that.
+#define GX_RAW_TOKENS 768
+template <bool RAW>
 __device__ __forceinline__ void gx_request(gx_set &st, const v4u *xhr, size_t xb, const uint16_t *dcol, uint32_t dm,
                                            uint32_t blk, uint32_t r64) {
     const v4u *p = xhr + blk * xb;
@@ -4496,15 +4503,22 @@ __device__ __forceinline__ void gx_request(gx_set &st, const v4u *xhr, size_t xb
     st.x[1] = p[r64];
     st.x[2] = p[4];
     st.x[3] = p[r64 + 4];
-    st.d = dcol[(size_t)blk * dm];
+    st.d = RAW ? (uint32_t)*(const u16_a1 *)(dcol + (size_t)blk * dm) : (uint32_t)dcol[(size_t)blk * dm];
 }
 // The thread's row weights of 4 consecutive blocks (one 128-byte line when
 // aligned), requested together: a row's blocks are K bytes apart from the
 // next row's, so a request per block would touch every line four times.
+template <bool RAW>
 __device__ __forceinline__ void gx_request_w4(v4u (&w)[8], const v4u *wrow, uint32_t blk, uint32_t kl) {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const uint32_t b = min(blk + j, kl);
+        if (RAW) {
+            const uint8_t *p = (const uint8_t *)wrow + (size_t)b * 34 + 2;
+            w[2 * j] = *(const v4u_a1 *)p;
+            w[2 * j + 1] = *(const v4u_a1 *)(p + 16);
+            continue;
+        }
         w[2 * j] = wrow[b * 2];
         w[2 * j + 1] = wrow[b * 2 + 1];
     }
@@ -4551,7 +4565,7 @@ __device__ __forceinline__ void gx_consume(f32x4 (&acc)[4][WT], uint16_t (&xt)[2
     __syncthreads();
 }
 
-template <int EPI, int NS, int CW>
+template <int EPI, int NS, int CW, bool RAW = false>
 __global__ void __launch_bounds__((CW + 4) * 64) __attribute__((amdgpu_waves_per_eu((CW + 4) / 4, (CW + 4) / 4)))
 k_gemm_q8_wide(const uint16_t *xs, const int8_t *qs, const uint16_t *d, float *Y, uint32_t N, uint32_t M,
                uint32_t K, uint32_t ldy, uint64_t ysplit, uint32_t boff) {
@@ -4578,8 +4592,9 @@ k_gemm_q8_wide(const uint16_t *xs, const int8_t *qs, const uint16_t *d, float *Y
         const size_t xb = (size_t)N * 8;
         const uint32_t r64 = (xn1 - xn0) * 8;                              // token p/4+64, in 16-byte units
         const uint32_t wrow_i = min(m0 + pt, M - 1);
-        const v4u *wrow = (const v4u *)(qs + (size_t)wrow_i * K);          // block s: wrow[2 s], wrow[2 s + 1]
-        const uint16_t *dcol = d + wrow_i;
+        const v4u *wrow = (const v4u *)(qs + (size_t)wrow_i * (RAW ? (size_t)nblk * 34 : (size_t)K));   // block s: wrow[2 s], wrow[2 s + 1]
+        const uint16_t *dcol = RAW ? (const uint16_t *)wrow : d + wrow_i;
+        const uint32_t dm = RAW ? 17 : M;
         // X and the scale per block in NS sets (block b in set (b - kb0) % NS);
         // weights per 4 blocks in two batches (block b in batch ((b - kb0) / 4) % 2,
         // slot (b - kb0) % 4), the next batch requested 4 steps before its first
@@ -4588,10 +4603,10 @@ k_gemm_q8_wide(const uint16_t *xs, const int8_t *qs, const uint16_t *d, float *Y
         gx_set g[NS];
         v4u wb[2][8];
         const uint32_t kl = kb1 - 1;
-        gx_request_w4(wb[0], wrow, kb0, kl);
-        gx_request_w4(wb[1], wrow, kb0 + 4, kl);
+        gx_request_w4<RAW>(wb[0], wrow, kb0, kl);
+        gx_request_w4<RAW>(wb[1], wrow, kb0 + 4, kl);
 #pragma unroll
-        for (int u = 0; u < NS - 1; u++) gx_request(g[u], xhr, xb, dcol, M, min(kb0 + u, kl), r64);
+        for (int u = 0; u < NS - 1; u++) gx_request<RAW>(g[u], xhr, xb, dcol, dm, min(kb0 + u, kl), r64);
         __builtin_amdgcn_sched_barrier(0);
         gx_stage(g[0], wb[0][0], wb[0][1], xt[0], wq[0], wd[0], pt, xo0, xo1);
         __syncthreads();
@@ -4602,9 +4617,9 @@ k_gemm_q8_wide(const uint16_t *xs, const int8_t *qs, const uint16_t *d, float *Y
                 // after a batch's last block is staged (steps 2 and 6) the
                 // batch 8 blocks on into it; stage block s+u+1 into the buffer
                 // step s+u does not read
-                gx_request(g[(u + NS - 1) % NS], xhr, xb, dcol, M, min(s + u + NS - 1, kl), r64);
-                if (u == 3) gx_request_w4(wb[0], wrow, s + 8, kl);
-                if (u == 7) gx_request_w4(wb[1], wrow, s + 12, kl);
+                gx_request<RAW>(g[(u + NS - 1) % NS], xhr, xb, dcol, dm, min(s + u + NS - 1, kl), r64);
+                if (u == 3) gx_request_w4<RAW>(wb[0], wrow, s + 8, kl);
+                if (u == 7) gx_request_w4<RAW>(wb[1], wrow, s + 12, kl);
                 __builtin_amdgcn_sched_barrier(0);
                 const uint32_t nbuf = (u & 1) ^ 1, b = ((u + 1) >> 2) & 1, j = (u + 1) & 3;
                 gx_stage(g[(u + 1) % NS], wb[b][2 * j], wb[b][2 * j + 1], xt[nbuf], wq[nbuf], wd[nbuf], pt, xo0, xo1);
@@ -5026,7 +5041,8 @@ extern "C" hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s) {
             hipLaunchKernelGGL(k_split_bf16, dim3(sg), dim3(TPB), 0, s, a->X, a->ldx, a->N, a->K, a->xs);
         }
         const int kind = gemm_kind();
-        if (a->N <= 16 * GF_NT_MAX && (kind == GEMM_WIDE || a->raw)) {
+        if (a->raw && (kind != GEMM_WIDE || epi != SGK_EPI_STORE)) return hipErrorInvalidValue;
+        if (a->N <= 16 * GF_NT_MAX && kind == GEMM_WIDE) {
             // three workgroups per CU, at least 16 blocks of K each, partials that fit (the
             // fused reduce is built for these counts): the 5120 x 17408 product of 40 tokens
             // took 52 us in 8 splits, 40 in 12, 46 in 16
@@ -5040,13 +5056,12 @@ extern "C" hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s) {
                                       : few_launch<SGK_EPI_STORE, false>(a, a->part, a->M, ys, S, s);
                 return e != hipSuccess ? e : splitk_finish(a, S, epi, Yo, s);
             }
-            if (a->raw) return epi == SGK_EPI_STORE ? few_launch<SGK_EPI_STORE, true>(a, a->Y, a->ldy, 0, 1, s) : hipErrorInvalidValue;
+            if (a->raw) return few_launch<SGK_EPI_STORE, true>(a, a->Y, a->ldy, 0, 1, s);
             if (epi == SGK_EPI_ADD) return few_launch<SGK_EPI_ADD, false>(a, a->Y, a->ldy, 0, 1, s);
             if (epi == SGK_EPI_SWIGLU) return few_launch<SGK_EPI_SWIGLU, false>(a, a->Y, a->ldy, 0, 1, s);
             if (epi == SGK_EPI_SWIGLU_XS) return few_launch<SGK_EPI_SWIGLU_XS, false>(a, Yo, a->ldy, 0, 1, s);
             return few_launch<SGK_EPI_STORE, false>(a, a->Y, a->ldy, 0, 1, s);
         }
-        if (a->raw) return hipErrorInvalidValue;
         const uint32_t TM = kind == GEMM_WIDE ? GX_TM : GM_TM;
         const uint32_t mb = (a->M + TM - 1) / TM, nb = (a->N + GM_TN - 1) / GM_TN;
         const uint32_t grid = 8 * gm_per_xcd(mb, nb), nblk = a->K / 32, tiles = mb * nb;
@@ -5061,7 +5076,10 @@ extern "C" hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s) {
         const uint32_t gtpb = kind == GEMM_PLAIN ? TPB : kind == GEMM_WIDE ? (GX_CW + 4) * 64 : GW_TPB;
 #define GL(E, G, Yp, LDY, YS, BOFF)                                                                             \
         do {                                                                                                   \
-            if (kind == GEMM_WIDE)                                                                              \
+            if (a->raw)                                                                                         \
+                hipLaunchKernelGGL((k_gemm_q8_wide<(E) == SGK_EPI_TILE ? SGK_EPI_TILE : SGK_EPI_STORE, GW_NS, GX_CW, true>), G, \
+                                   dim3(gtpb), 0, s, a->xs, (const int8_t *)a->raw, a->dt, Yp, a->N, a->M, a->K, LDY, YS, BOFF); \
+            else if (kind == GEMM_WIDE)                                                                         \
                 hipLaunchKernelGGL((k_gemm_q8_wide<E, GW_NS, GX_CW>), G, dim3(gtpb), 0, s, a->xs, a->qs, a->dt, Yp, a->N, \
                                    a->M, a->K, LDY, YS, BOFF);                                                 \
             else if (kind == GEMM_WS)                                                                           \
@@ -5123,7 +5141,8 @@ extern "C" hipError_t sgk_gemm_q8(const float *X, const int8_t *qs, const uint16
     a.raw = raw;
     return sgk_gemm(&a, s);
 }
-extern "C" uint32_t sgk_gemm_raw_tokens(void) { return 16 * GF_NT_MAX; }
+extern "C" uint32_t sgk_gemm_few_tokens(void) { return 16 * GF_NT_MAX; }
+extern "C" int sgk_gemm_takes_raw(uint32_t N) { return gemm_kind() == GEMM_WIDE && N <= GX_RAW_TOKENS; }
 
 // ---------------------------------------------------------------------------
 // Measurement kernels: a plain streaming read (16-byte non-temporal loads, a
