@@ -723,8 +723,9 @@ sg_err sg_gpu_run_delta_multi(sg_gpu *g, void *S, void *qkv, void *out, void *ga
  *         updated in place;
  *   out   [value_dim]                     silu(z) * rmsnorm(y, ssm_norm).
  * p: [0]=dk [1]=dv [2]=n_v [3]=n_k [4]=ksize [5]=tiled [6]=ssm_a is -exp(A_log)
- * [7]=eps bits. conv_dim = 2 n_k dk + n_v dv. head_v_dim <= 128 (one
- * workgroup per value head, the decode default). */
+ * [7]=eps bits. conv_dim = 2 n_k dk + n_v dv. head_v_dim <= 128; a multiple
+ * of SGK_GDN_BLOCKS runs the decode's form on the tail itself, any other one
+ * workgroup per value head with the tail copied to a ring and back. */
 /* SURGE_DELTA_SCAN, the prefill DeltaNet scan's form: mfma (default) or seq.
  * Any other value is refused, not ignored, so an A/B of scan forms never
  * measures one it did not name. */

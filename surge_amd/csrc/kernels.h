@@ -137,13 +137,6 @@ typedef struct {
     float *m, *s, *acc;         /* partials */
     float *out;                 /* combine output [ntok][n_heads*hd] */
     const float *gate;          /* combine: the output gate's rows, or NULL */
-    uint32_t gate_tok, gate_stride; /* its strides per token and head (0: as q) */
-    /* prep: where the projection's rows (q|gate|k|v) are read when not in place:
-     * token z's at src + z*src_tok, query head h's at + h*src_stride, k and v
-     * after the last head's; q is then written to a->q (NULL: q holds the rows
-     * and is normalised in place) */
-    const float *src;
-    uint32_t src_tok, src_stride;
     const sgk_step *steps;
     uint32_t n_heads, n_kv, hd, rope_dim, q_stride, q_tok, out_tok;
     uint32_t seq, n_splits, max_splits, ntok;
@@ -167,6 +160,16 @@ typedef struct {
      * grid's y is n_heads. Each head's arithmetic is the same as in the
      * group-shared form, so both give the same bytes. */
     int per_head;
+    /* The last fields are the chunk path's only, behind what the decode kernels
+     * read of their arguments. Strides of the gate's rows per token and head
+     * (0: as q). */
+    uint32_t gate_tok, gate_stride;
+    /* prep: where the projection's rows (q|gate|k|v) are read when not in place:
+     * token z's at src + z*src_tok, query head h's at + h*src_stride, k and v
+     * after the last head's; q is then written to a->q (NULL: q holds the rows
+     * and is normalised in place) */
+    const float *src;
+    uint32_t src_tok, src_stride;
 } sgk_attn;
 
 /* q_norm/k_norm + RoPE on each head, K and V stored f16 at each token's

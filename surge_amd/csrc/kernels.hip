@@ -2154,7 +2154,7 @@ __global__ void __launch_bounds__(TPB) k_attn_combine(sgk_attn a) {
     const float *mh = a.m + zoff + (size_t)h * ns, *sh = a.s + zoff + (size_t)h * ns;
     const float4 *acc = (const float4 *)(a.acc + (zoff + (size_t)h * ns) * HD);
     float *oh = a.out + (size_t)z * a.out_tok + (size_t)h * HD;
-    const float *gate = a.gate ? a.gate + (size_t)z * a.gate_tok + (size_t)h * a.gate_stride : NULL;
+    const float *gate = a.gate ? a.gate + (size_t)z * a.q_tok + (size_t)h * a.q_stride : NULL;   // (the launcher's: the gate's strides)
     // every load that does not depend on the merge weights goes out first:
     // this thread's first split's max and sum, and its first PFX rows of acc
     const uint32_t c = t % C4, kg = t / C4;
@@ -2546,7 +2546,12 @@ extern "C" hipError_t sgk_attn_combine(const sgk_attn *a, hipStream_t s) {
     if (!a->n_heads || !a->ntok) return hipSuccess;
     if (!a->steps && a->n_splits > 1024) return hipErrorInvalidValue;
     dim3 grid(a->n_heads, a->ntok);
-#define HDCASE(H) case H: hipLaunchKernelGGL(k_attn_combine<H>, grid, dim3(TPB), 0, s, kv_resolved(a)); break
+    // the combine reads no q, so the gate's strides go in q's place: with them behind the
+    // other fields a decode call of 512 keys took 20.7 us, not 20.3
+    sgk_attn k = kv_resolved(a);
+    k.q_tok = k.gate_tok;
+    k.q_stride = k.gate_stride;
+#define HDCASE(H) case H: hipLaunchKernelGGL(k_attn_combine<H>, grid, dim3(TPB), 0, s, k); break
     switch (a->hd) {
         HDCASE(16); HDCASE(32); HDCASE(64); HDCASE(128); HDCASE(256);
     default: return hipErrorInvalidValue;
