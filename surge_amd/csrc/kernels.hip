@@ -565,7 +565,7 @@ __device__ __forceinline__ void raw_load(gemv_chunk<2> &ch, const uint8_t *w, ui
         const uint8_t *p = w + (size_t)min(r0 + r, rows - 1) * rb + (size_t)(cc >> 1) * 34;
         const v4u_a2 v = *(const v4u_a2 *)(p + 2 + 16 * (cc & 1));
         ch.q[r] = make_uint4(v.x, v.y, v.z, v.w);
-        ch.d[r] = c < nch ? *(const uint16_t *)p : (uint16_t)0;
+        ch.d[r] = *(const uint16_t *)p;
     }
 }
 
@@ -586,7 +586,8 @@ __global__ void __launch_bounds__(TPB) k_gemv_raw(sgk_gemv a, const uint8_t *w) 
         float acc[2] = {0.0f, 0.0f};
         for (uint32_t c = lane;;) {
 #pragma unroll
-            for (int u = 0; u < RAW_U; u++) gemv_fma<2, false>(acc, ch[u], xs, min(c + 64 * u, nch - 1));
+            for (int u = 0; u < RAW_U; u++)
+                if (c + 64 * u < nch) gemv_fma<2, false>(acc, ch[u], xs, c + 64 * u);   // no 0 * x past the row: x may be infinite
             c += 64 * RAW_U;
             const bool more = c - lane < nch;
             // the row's next half blocks, or the next row pair's first

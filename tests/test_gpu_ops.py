@@ -125,6 +125,24 @@ def test_gemv_q8_on_blocks(gpu, rows, cols, off):
     assert_close(yb.array, oracle_matvec_q8(raw, x, rows, cols), 1e-5)
 
 
+@pytest.mark.parametrize("cols", [32, 1056, 2080, 5120, 17408])
+@pytest.mark.parametrize("v", [np.inf, -np.inf, 3e38])
+def test_gemv_q8_infinite_products_stay_infinite(gpu, cols, v):
+    """An infinity (or a value whose products overflow) in x's last 16 columns
+    at widths that leave lanes past the row's end: the row sums are infinities
+    of the products' sign, as in the oracle, and NaN nowhere (a lane without a
+    half block must not multiply x by a zero)."""
+    rows = 5
+    rng = np.random.default_rng(cols)
+    raw = q8_matrix(rng, rows, cols, sigma=1.0).reshape(rows, cols // 32, 34)
+    raw[:, -1, :2] = np.full(rows, 2.0, np.float16).view(np.uint8).reshape(rows, 2)
+    raw[:, -1, 2:] = np.array([100, -100, 7, -7, 127], np.int8).view(np.uint8)[:, None]
+    x = rng.standard_normal(cols).astype(np.float32)
+    x[-3] = v
+    got = gpu_matvec_q8(gpu, raw.reshape(-1), x, rows, cols)
+    assert np.array_equal(got, np.sign(v) * np.array([np.inf, -np.inf, np.inf, -np.inf, np.inf], np.float32))
+
+
 def test_gemv_f32(gpu):
     rng = np.random.default_rng(3)
     rows, cols = 50, 24
