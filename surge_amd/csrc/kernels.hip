@@ -1003,8 +1003,11 @@ extern "C" hipError_t sgk_gemv_raw(const uint8_t *w, uint32_t rows, uint32_t col
     const size_t lds = (size_t)cols * 4;
     hipError_t e = allow_lds((const void *)k_gemv_raw, lds);
     if (e != hipSuccess) return e;
-    // resident workgroups only (VGPRs allow 8 a CU): each walks row pairs with a grid stride
-    const uint32_t per = min((uint32_t)(163840 / lds), 8u), groups = (rows + 1) / 2;
+    // resident workgroups only, each walking row pairs with a grid stride: the LDS
+    // for x and, up to 8192 columns, five a CU. The registers (66) allow seven;
+    // 17408 x 5120 took 40.0 us a call with five, 42.1 with seven and 43.6 with
+    // eight, of which one in eight waits for a place; 12288 x 5120 32.7, 33.7, 33.6
+    const uint32_t per = min((uint32_t)(163840 / lds), 5u), groups = (rows + 1) / 2;
     const uint32_t blocks = min((groups + 3) / 4, (uint32_t)device_cus() * per);
     hipLaunchKernelGGL(k_gemv_raw, dim3(blocks), dim3(TPB), lds, s, a, w);
     return hipGetLastError();
