@@ -29,6 +29,13 @@ extern "C" {
 #define SGK_G
 #endif
 
+/* Rules that both passes evaluate. */
+#ifdef __HIPCC__
+#define SGK_HD __host__ __device__
+#else
+#define SGK_HD
+#endif
+
 /* Per-token step descriptor, read by every position-dependent kernel so one
  * captured HIP graph serves every decode step. */
 typedef struct {
@@ -236,6 +243,13 @@ hipError_t sgk_gdn_step(const sgk_gdn *a, hipStream_t s);
  * moved on in place; no step descriptor), RMSNormGated finished into out; dv a
  * multiple of SGK_GDN_BLOCKS, ss scratch. */
 hipError_t sgk_gdn_step_tail(const sgk_gdn *a, hipStream_t s);
+
+/* The row of a caller's conv tail [keep][conv_dim] (keep = ksize - 1, oldest
+ * first) that holds the input of position z < 0 before a chunk, or -1: the
+ * tail has no such row, and nothing may be read there (with keep 0 the tail is
+ * empty and what lies at its address is the state, which may be shorter than
+ * conv_dim). */
+SGK_HD static inline int sgk_tail_row(uint32_t keep, int z) { return (int)keep + z >= 0 ? (int)keep + z : -1; }
 
 /* The DeltaNet layer over a prefill chunk of ntok tokens (a->step holds the
  * chunk's descriptors, a->in the chunk's GEMM rows at in_stride, a->y the

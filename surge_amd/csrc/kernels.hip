@@ -2747,10 +2747,11 @@ __device__ __forceinline__ void gdn_step_body(const sgk_gdn &a, uint32_t h, uint
         cw.y = a.conv_w[(size_t)c * a.ksize + min(1u, keep)];
         cw.z = a.conv_w[(size_t)c * a.ksize + min(2u, keep)];
         cw.w = a.conv_w[(size_t)c * a.ksize + min(3u, keep)];
-        // a tail has keep rows (with none, the state behind it is read and not used)
-        rs.x = a.ring[c];
-        rs.y = a.ring[(size_t)(TAIL ? min(1u, max(keep, 1u) - 1) : 1) * cd + c];
-        rs.z = a.ring[(size_t)(TAIL ? min(2u, max(keep, 1u) - 1) : 2) * cd + c];
+        // a tail has keep rows; with none, the row read (and not used) is the input's
+        const auto *past = TAIL && keep == 0 ? a.in : a.ring;
+        rs.x = past[c];
+        rs.y = past[(size_t)(TAIL ? min(1u, max(keep, 1u) - 1) : 1) * cd + c];
+        rs.z = past[(size_t)(TAIL ? min(2u, max(keep, 1u) - 1) : 2) * cd + c];
         rs.w = TAIL ? 0.0f : a.ring[(size_t)3 * cd + c];
     };
     const uint32_t ch0 = chan(min(t, nch - 1)), ch1 = chan(min(t + GDN_TPB, nch - 1));
@@ -3118,9 +3119,9 @@ __global__ void __launch_bounds__(TPB) k_conv_chunk(const float *in, uint32_t in
             const int z = (int)z0 + i - 3;
             const uint32_t zc = (uint32_t)min(max(z, 0), (int)ntok - 1);
             x[i] = in[(size_t)zc * in_stride + ch];
-            if (i < 3 && z0 == 0) {      // z < 0; no tail row keep + z (z < -keep): not used
-                const uint32_t r = TAIL ? (uint32_t)max((int)keep + z, 0) : (pos0 + 4 + (uint32_t)z) & 3;
-                x[i] = ring[(size_t)r * cd + ch];
+            if (i < 3 && z0 == 0) {      // z < 0; a tail without the row: x[i] is not used
+                const int r = TAIL ? sgk_tail_row(keep, z) : (int)((pos0 + 4 + (uint32_t)z) & 3);
+                if (!TAIL || r >= 0) x[i] = ring[(size_t)r * cd + ch];
             }
         }
 #pragma unroll

@@ -537,11 +537,13 @@ def test_gdn_step_on_tail_edges(gpu, nv, nk, dk, dv, ks, tiled):
 
 
 @pytest.mark.parametrize("nv,nk,dk,dv,ks,tiled,n1,n2", [(48, 16, 128, 128, 4, True, 215, 1), (2, 1, 64, 64, 1, True, 3, 2),
-                                                        (3, 3, 128, 256, 3, True, 1, 17)])
+                                                        (3, 3, 128, 256, 3, True, 1, 17), (16, 16, 256, 1, 1, True, 5, 1),
+                                                        (4, 4, 32, 2, 1, True, 1, 18), (2, 1, 64, 1, 2, True, 1, 2)])
 def test_gdn_chunk_forms(gpu, nv, nk, dk, dv, ks, tiled, n1, n2):
     """The chunk conv with sixteen tokens per thread and with four, no tail, a
-    chunk shorter than the tail (old rows stay), and the float4 norm with rows
-    that do not fill a workgroup."""
+    chunk shorter than the tail (old rows stay), the float4 norm with rows that
+    do not fill a workgroup, and states shorter than a conv row (one or two
+    value rows a head), which an empty tail's row must not be read from."""
     test_gdn_prefill_chunk_vs_oracle(gpu, nv, nk, dk, dv, ks, tiled, n1, n2)
 
 

@@ -172,6 +172,45 @@ def test_gpu_init_fails_cleanly_without_a_device():
         assert b"no HIP device" in err.msg
 
 
+# ---------------------------------------------------------------- rules the kernels share with the host
+
+def test_conv_tail_rows_stay_inside_the_state():
+    """The row that the DeltaNet chunk's conv reads for each of the three
+    positions before the chunk (sgk_tail_row, compiled here for the host), over
+    the shapes the chunk call accepts: the row that holds the position, inside
+    the tail of the caller's [ksize-1][conv_dim] + n_v dv dk floats, and none
+    where the tail has no such row. With ksize 1 the tail is empty and the
+    state may be shorter than a row of conv_dim."""
+    import subprocess
+    src = r"""
+#include <stdio.h>
+#include "kernels.h"
+int main(void) {
+    const uint32_t dks[] = {32, 64, 128, 256}, dvs[] = {1, 2, 3, 4, 16, 128};
+    int shorter = 0;
+    for (uint32_t ks = 1; ks <= 4; ks++)
+        for (int a = 0; a < 4; a++) for (int b = 0; b < 6; b++)
+            for (uint32_t nk = 1; nk <= 16; nk++) for (uint32_t f = 1; f <= 3; f++) {
+                const uint64_t keep = ks - 1, nv = nk * f, cd = 2ull * nk * dks[a] + nv * dvs[b];
+                const uint64_t floats = keep * cd + nv * dvs[b] * dks[a];
+                shorter += floats < cd;
+                for (int z = -3; z < 0; z++) {
+                    const int r = sgk_tail_row(ks - 1, z);
+                    if (r < 0) { if ((int)keep + z >= 0) return 1; continue; }
+                    if (r != (int)keep + z || (r + 1) * cd > keep * cd || (r + 1) * cd > floats) return 2;
+                }
+            }
+    return shorter ? 0 : 3;
+}
+"""
+    with tempfile.TemporaryDirectory() as d:
+        c, exe = os.path.join(d, "u.c"), os.path.join(d, "u")
+        open(c, "w").write(src)
+        inc = os.path.join(os.path.dirname(S.LIB_PATH), "csrc")
+        subprocess.check_call(["gcc", "-std=c11", "-D__HIP_PLATFORM_AMD__", "-I", inc, "-I", "/opt/rocm/include", c, "-o", exe])
+        assert subprocess.call([exe]) == 0
+
+
 # ---------------------------------------------------------------- the C ABI against the reference header
 
 REF_HEADER = "/root/reference/surge.h"
