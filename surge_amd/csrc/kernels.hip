@@ -3239,7 +3239,14 @@ __device__ __forceinline__ void dc_load(dcregs<DK, ROWS> &r, const sgk_gdn &a, c
     // v: token t/VTT, rows j0 + 4*(t%VTT) .. +3
     const uint32_t vz = t / C::VTT, vr = j0 + (t % C::VTT) * 4;
     const float *vp = conv_out + (size_t)min(z0 + vz, ntok - 1) * a.conv_dim + 2 * key_dim + (size_t)h * a.dv + vr;
-    r[C::NV4] = (vz < (uint32_t)C::DCT && vr < a.dv) ? *(const f32x4 *)vp : (f32x4){0.f, 0.f, 0.f, 0.f};
+    r[C::NV4] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (vz < (uint32_t)C::DCT && vr + 4 <= a.dv) {
+        r[C::NV4] = *(const f32x4 *)vp;
+    } else if (vz < (uint32_t)C::DCT) {         // dv % 4: the last rows one by one (the last head's end the caller's buffer)
+#pragma unroll
+        for (uint32_t e = 0; e < 3; e++)
+            if (vr + e < a.dv) r[C::NV4][e] = vp[e];
+    }
 }
 
 template <int DK, int ROWS>

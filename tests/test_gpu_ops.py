@@ -861,6 +861,15 @@ def test_delta_chunk_chunked_form_vs_sequential_oracle(gpu, monkeypatch, scan, n
     assert_close(Sgot, Swant)
 
 
+@pytest.mark.parametrize("nv,nk,dk,dv,nt", [(2, 1, 64, 1, 17), (3, 3, 32, 6, 16), (4, 2, 256, 19, 33)])
+def test_delta_chunk_rows_off_a_vector(gpu, nv, nk, dk, dv, nt):
+    """Value rows that no float4 divides: the last rows of a head are loaded one
+    by one, and the last head's end where the caller's rows end."""
+    got, Sgot, want, Swant = _delta_chunk_case(gpu, nv, nk, dk, dv, nt, seed=5 + dv)
+    assert_close(got, want)
+    assert_close(Sgot, Swant)
+
+
 def test_delta_chunk_chunked_form_tiny_decays(gpu, monkeypatch):
     """Decays down to 1e-30 per token: the chunked form's decay products
     (plain products over a 16-token block) underflow to exact zeros instead
