@@ -2698,7 +2698,7 @@ __device__ __forceinline__ uint32_t rows_lane(uint32_t r) {   // a lane holding 
 // rows' squared readouts, with no synchronisation between blocks.
 // TAIL: the conv's past inputs are the caller's tail, oldest first
 // (a.ring = [ksize-1][conv_dim]), which is only read here (k_gdn_finish moves
-// it on); no position is needed.
+// it on); no position is needed. The readouts go to a.out as they are.
 template <int DK, int RW, int NB, int GDN_TPB, bool TAIL>
 __device__ __forceinline__ void gdn_step_body(const sgk_gdn &a, uint32_t h, uint32_t jb) {
     constexpr int GDN_NB = NB;
@@ -2757,8 +2757,8 @@ __device__ __forceinline__ void gdn_step_body(const sgk_gdn &a, uint32_t h, uint
     const uint32_t ch0 = chan(min(t, nch - 1)), ch1 = chan(min(t + GDN_TPB, nch - 1));
     conv_loads(cx0, cw0, rs0, ch0);
     conv_loads(cx1, cw1, rs1, ch1);
-    const float zraw = a.z[(size_t)h * dv + min(max(t, jlo), jhi - 1)];
-    const float nwt = a.norm_w[min(t, dv - 1)];   // needed last, loaded early
+    const float zraw = TAIL ? 0.0f : a.z[(size_t)h * dv + min(max(t, jlo), jhi - 1)];
+    const float nwt = TAIL ? 0.0f : a.norm_w[min(t, dv - 1)];   // needed last, loaded early
     const float *bb = a.in + cd + a.n_v * dv, *aa = bb + a.n_v;
     const float gb = bb[h], ga = aa[h], gA = a.ssm_a[h], gdt = a.dt_bias[h];
     const uint32_t j0 = jlo + wave * RW;
@@ -2892,7 +2892,7 @@ __device__ __forceinline__ void gdn_step_body(const sgk_gdn &a, uint32_t h, uint
         for (int w = 0; w < NW; w++) sb += red[w];
         a.ss[(size_t)h * GDN_NB + jb] = sb;
     }
-    if (t >= jlo && t < jhi) a.out[(size_t)h * dv + t] = silu(zj) * (ysh[t] * nwt);
+    if (t >= jlo && t < jhi) a.out[(size_t)h * dv + t] = TAIL ? ysh[t] : silu(zj) * (ysh[t] * nwt);
 }
 
 template <int DK, int RW, int NB, int GDN_TPB, bool TAIL = false>
@@ -2911,9 +2911,11 @@ __device__ __forceinline__ void conv_tail(const float *in, uint32_t in_stride, f
                                                     : in[(size_t)(ntok + j - keep) * in_stride + ch];
 }
 
-// What a step on the caller's tail leaves to do: each head's RMS factor from
-// its row blocks' sums of squares (added in block order, as the gated GEMV
-// prologue does) applied to its outputs, and the tail moved on by one input.
+// What a step on the caller's tail leaves to do: RMSNormGated of the readouts
+// in a.out with each head's factor from its row blocks' sums of squares (added
+// in block order, as the gated GEMV prologue does), and the tail moved on by
+// one input. The factor goes to the readout first, as in the one-block form:
+// silu(z) (y w) of large z and y overflows where the normed product does not.
 // Thread i takes output i and channel i.
 __global__ void __launch_bounds__(TPB) k_gdn_finish(sgk_gdn a) {
     const uint32_t i = blockIdx.x * TPB + threadIdx.x;
@@ -2922,7 +2924,7 @@ __global__ void __launch_bounds__(TPB) k_gdn_finish(sgk_gdn a) {
         float tot = 0.0f;
 #pragma unroll
         for (uint32_t b = 0; b < SGK_GDN_BLOCKS; b++) tot += a.ss[h * SGK_GDN_BLOCKS + b];
-        a.out[i] *= 1.0f / sqrtf(tot / (float)a.dv + a.eps);
+        a.out[i] = silu(a.z[i]) * ((a.out[i] * (1.0f / sqrtf(tot / (float)a.dv + a.eps))) * a.norm_w[i % a.dv]);
     }
     if (i < a.conv_dim) conv_tail((const float *)a.in, 0, (float *)a.ring, 1, a.conv_dim, a.ksize - 1, i);
 }

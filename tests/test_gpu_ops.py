@@ -536,6 +536,26 @@ def test_gdn_step_on_tail_edges(gpu, nv, nk, dk, dv, ks, tiled):
     test_gdn_decode_step_vs_oracle(gpu, nv, nk, dk, dv, ks, tiled)
 
 
+@pytest.mark.parametrize("dv", [5, 128])
+def test_gdn_step_large_gate_and_state(gpu, dv):
+    """A readout near 1e16 and a gate near 1e25: their product overflows, the
+    gated norm does not. Both forms (dv 128 on the tail, 5 through the ring)
+    within 1e-3 of the oracle."""
+    nv, nk, dk, ks, eps = 4, 2, 64, 4, 1e-6
+    rng = np.random.default_rng(dv)
+    cd, vd = 2 * nk * dk + nv * dv, nv * dv
+    w = np.concatenate([rng.standard_normal(cd * ks) * 0.5, -np.exp(rng.uniform(-1, 1, nv)),
+                        rng.uniform(-0.5, 0.5, nv), 1.0 + 0.1 * rng.standard_normal(dv)]).astype(np.float32)
+    state = np.concatenate([rng.standard_normal((ks - 1) * cd), rng.standard_normal(vd * dk) * 1e18]).astype(np.float32)
+    inp = rng.standard_normal(cd + vd + 2 * nv).astype(np.float32)
+    inp[cd:cd + vd] *= 1e25
+    ib, wb, sb, ob = gpu.buf(inp), gpu.buf(w), gpu.buf(state.copy()), gpu.buf(np.zeros(vd, np.float32))
+    gpu.gdn_step(ib, wb, sb, ob, [dk, dv, nv, nk, ks, 1, 1, S.fbits(eps)])
+    want, _ = oracle_gdn_step(inp, w, state, dk, dv, nv, nk, ks, True, eps)
+    assert np.isfinite(want).all()
+    assert_close(ob.array, want)
+
+
 @pytest.mark.parametrize("nv,nk,dk,dv,ks,tiled,n1,n2", [(48, 16, 128, 128, 4, True, 215, 1), (2, 1, 64, 64, 1, True, 3, 2),
                                                         (3, 3, 128, 256, 3, True, 1, 17), (16, 16, 256, 1, 1, True, 5, 1),
                                                         (4, 4, 32, 2, 1, True, 1, 18), (2, 1, 64, 1, 2, True, 1, 2)])
