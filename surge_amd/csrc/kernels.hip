@@ -4822,10 +4822,15 @@ k_gemm_q8_few(const uint16_t *xs, const void *w, const uint16_t *d, float *Y, ui
     __syncthreads();
     uint32_t buf = 0;
     for (uint32_t s = kb0; s < kb1; s += 4) {
-        store_w(wv);                            // (this wave's LDS operations run in order)
+        load_x(min(s + XB, kl));                // (before the wait for the weights)
+        store_w(wv);
+        // other lanes of the wave read them: the LDS runs a wave's operations in order, and the
+        // fence (no instruction) keeps the compiler from moving the reads above the stores
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int o = 0; o < 4; o += XB, buf ^= 1) {
-            load_x(min(s + o + XB, kl));
+            if (o) load_x(min(s + o + XB, kl));
             __builtin_amdgcn_sched_barrier(0);
             if (o == 0) load_w(wv, min(s + 4, kl));
             __builtin_amdgcn_sched_barrier(0);
