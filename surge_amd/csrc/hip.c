@@ -403,8 +403,9 @@ sg_err sg_gpu_run_op(sg_gpu *g, const char *kernel, void *a, void *b, void *out,
         sgk_gemv ga = {0};
         ga.rows = rows; ga.cols = cols; ga.x = DEV(b); ga.y = DEV(out);
         ga.pro = SGK_PRO_NONE; ga.epi = SGK_EPI_STORE;
-        if (q8 && !((uintptr_t)DEV(a) & 1)) return finish(g, sgk_gemv_raw(DEV(a), rows, cols, DEV(b), DEV(out), s), outs, 1);
-        if (q8) {               /* blocks at an odd address: repacked first */
+        if (q8 && !getenv("SURGE_GEMV") && !((uintptr_t)DEV(a) & 1))
+            return finish(g, sgk_gemv_raw(DEV(a), rows, cols, DEV(b), DEV(out), s), outs, 1);
+        if (q8) {               /* repacked first: blocks at an odd address, and where SURGE_GEMV names a kernel */
             void *t;
             if (sg_failed(e = scratch(g, (uint64_t)rows * cols + (uint64_t)rows * (cols / 32) * 2 + 256, &t))) return e;
             ga.qs = t;

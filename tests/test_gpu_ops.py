@@ -143,6 +143,23 @@ def test_gemv_q8_infinite_products_stay_infinite(gpu, cols, v):
     assert np.array_equal(got, np.sign(v) * np.array([np.inf, -np.inf, np.inf, -np.inf, np.inf], np.float32))
 
 
+@pytest.mark.parametrize("rows,cols", [(3, 96), (4096, 4096), (1030, 2080), (700, 5120)])
+def test_gemv_q8_env_names_the_kernel(gpu, monkeypatch, rows, cols):
+    """SURGE_GEMV names a kernel on the planes, in the one-call matvec too.
+    k_gemv_q8 has the lanes, chunks and order of sums of the blocks' kernel, so
+    the same bits; k_gemv_bal (multiples of 1024 columns only) splits rows over
+    waves: other bits, within 1e-6 of the largest value."""
+    rng = np.random.default_rng(rows)
+    raw, x = q8_matrix(rng, rows, cols), rng.standard_normal(cols).astype(np.float32)
+    blocks = gpu_matvec_q8(gpu, raw, x, rows, cols)
+    monkeypatch.setenv("SURGE_GEMV", "q8")
+    assert np.array_equal(gpu_matvec_q8(gpu, raw, x, rows, cols), blocks)
+    monkeypatch.setenv("SURGE_GEMV", "bali")
+    bali = gpu_matvec_q8(gpu, raw, x, rows, cols)
+    assert_close(bali, blocks, 1e-6)
+    assert np.array_equal(bali, blocks) == (cols % 1024 != 0)
+
+
 def test_gemv_f32(gpu):
     rng = np.random.default_rng(3)
     rows, cols = 50, 24
