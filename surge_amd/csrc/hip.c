@@ -375,6 +375,19 @@ static sg_err scratch(sg_gpu *g, uint64_t bytes, void **out) {
 
 #define DEV(b) ((b) ? ((gbuf *)(b))->dev : NULL)
 
+/* SURGE_ONESHOT: the forms that the one-call products and layers run where
+ * they have one of their own: "call" (default), built for a caller's buffers
+ * (the file's blocks as they lie, a conv tail, rows read in place), or
+ * "model", the model's (weights repacked into planes, a position ring, rows
+ * prepared in place under a table from position 0), so that those kernels are
+ * checked one by one too. Any other value is refused. */
+static sg_err oneshot_env(bool *model) {
+    const char *v = getenv("SURGE_ONESHOT");
+    *model = v && !strcmp(v, "model");
+    if (v && !*model && strcmp(v, "call")) return errf("gpu: SURGE_ONESHOT='%s' must be call or model (default call)", v);
+    return SG_OK;
+}
+
 /* ---------------------------------------------------------------------
  * sg_gpu_run_op: the per-op oracle hooks (surge.h:666-762)
  * --------------------------------------------------------------------- */
@@ -389,7 +402,9 @@ sg_err sg_gpu_run_op(sg_gpu *g, const char *kernel, void *a, void *b, void *out,
     void *ins[3] = {a, b, out};
     void *outs[1] = {out};
     hipStream_t s = g->stream;
-    sg_err e;
+    bool model;
+    sg_err e = oneshot_env(&model);
+    if (sg_failed(e)) return e;
     const uint32_t n = p[0];
 
     if (!strcmp(kernel, "k_matvec_q8") || !strcmp(kernel, "k_matvec_f32")) {
@@ -403,9 +418,9 @@ sg_err sg_gpu_run_op(sg_gpu *g, const char *kernel, void *a, void *b, void *out,
         sgk_gemv ga = {0};
         ga.rows = rows; ga.cols = cols; ga.x = DEV(b); ga.y = DEV(out);
         ga.pro = SGK_PRO_NONE; ga.epi = SGK_EPI_STORE;
-        if (q8 && !getenv("SURGE_GEMV") && !((uintptr_t)DEV(a) & 1))
+        if (q8 && !model && !getenv("SURGE_GEMV") && !((uintptr_t)DEV(a) & 1))
             return finish(g, sgk_gemv_raw(DEV(a), rows, cols, DEV(b), DEV(out), s), outs, 1);
-        if (q8) {               /* repacked first: blocks at an odd address, and where SURGE_GEMV names a kernel */
+        if (q8) {               /* repacked first: also for blocks at an odd address, and where SURGE_GEMV names a kernel */
             void *t;
             if (sg_failed(e = scratch(g, (uint64_t)rows * cols + (uint64_t)rows * (cols / 32) * 2 + 256, &t))) return e;
             ga.qs = t;
@@ -514,7 +529,7 @@ sg_err sg_gpu_run_op(sg_gpu *g, const char *kernel, void *a, void *b, void *out,
             sg_failed(e = need(out, (uint64_t)N * M * 4, "Y"))) return e;
         if (sg_failed(e = push(ins, 3))) return e;
         void *t;
-        const bool raw = sgk_gemm_takes_raw(N);         /* else through the repacked planes */
+        const bool raw = !model && sgk_gemm_takes_raw(N);       /* else through the repacked planes */
         const uint64_t qb = raw ? 0 : ((uint64_t)M * K + 255) / 256 * 256, db = raw ? 0 : ((uint64_t)M * (K / 32) * 2 + 255) / 256 * 256;
         const uint64_t xb = ((uint64_t)N * K * 4 + 255) / 256 * 256, pc = (uint64_t)(N <= sgk_gemm_few_tokens() ? 12 : 4) * N * M;   /* split-K partials */
         if (sg_failed(e = scratch(g, qb + 2 * db + xb + pc * 4, &t))) return e;
@@ -725,8 +740,9 @@ sg_err sg_gpu_run_delta_multi(sg_gpu *g, void *S, void *qkv, void *out, void *ga
  *   out   [value_dim]                     silu(z) * rmsnorm(y, ssm_norm).
  * p: [0]=dk [1]=dv [2]=n_v [3]=n_k [4]=ksize [5]=tiled [6]=ssm_a is -exp(A_log)
  * [7]=eps bits. conv_dim = 2 n_k dk + n_v dv. head_v_dim <= 128; a multiple
- * of SGK_GDN_BLOCKS runs the decode's form on the tail itself, any other one
- * workgroup per value head with the tail copied to a ring and back. */
+ * of SGK_GDN_BLOCKS runs SGK_GDN_BLOCKS workgroups per value head on the tail
+ * itself; any other, and SURGE_ONESHOT=model, one workgroup per head with the
+ * tail copied to a position ring (the decode's) and back. */
 /* SURGE_DELTA_SCAN, the prefill DeltaNet scan's form: mfma (default) or seq.
  * Any other value is refused, not ignored, so an A/B of scan forms never
  * measures one it did not name. */
@@ -750,8 +766,9 @@ sg_err sg_gpu_run_gdn_step(sg_gpu *g, void *in, void *w, void *state, void *out,
     if (overlap(out, in) || overlap(out, w) || overlap(out, state) || overlap(state, in) || overlap(state, w))
         return (sg_err){"gpu: gdn_step: buffers must not overlap"};
     void *ins[3] = {in, w, state}, *outs[2] = {state, out};
-    if (sg_failed(e = push(ins, 3))) return e;
-    if (dv % SGK_GDN_BLOCKS == 0) {         /* on the tail itself; scratch: the row blocks' sums of squares */
+    bool model;
+    if (sg_failed(e = oneshot_env(&model)) || sg_failed(e = push(ins, 3))) return e;
+    if (dv % SGK_GDN_BLOCKS == 0 && !model) {         /* on the tail itself; scratch: the row blocks' sums of squares */
         void *ss;
         if (sg_failed(e = scratch(g, (uint64_t)nv * SGK_GDN_BLOCKS * 4, &ss))) return e;
         float *dst = DEV(state), *wp = DEV(w);
@@ -785,10 +802,12 @@ sg_err sg_gpu_run_gdn_step(sg_gpu *g, void *in, void *w, void *state, void *out,
     return finish(g, he, outs, 2);
 }
 
-/* The prefill path's DeltaNet layer core over a chunk of n tokens, with the
- * kernels prefill_chunk runs (sgk_gdn_chunk: the chunk conv with its q/k
- * norm, the conv ring, the gates and the delta-rule scan in the build's
- * default form; then the RMSNormGated rows) on caller buffers (no reference
+/* The prefill path's DeltaNet layer core over a chunk of n tokens, with
+ * prefill_chunk's kernels (sgk_gdn_chunk: the chunk conv with its q/k norm,
+ * the gates and the delta-rule scan in the build's default form, the conv's
+ * past inputs moved on; then the RMSNormGated rows) on caller buffers. The
+ * conv reads the caller's tail in place of prefill's position ring, and the
+ * norm writes f32 rows in place of the next product's split (no reference
  * counterpart: the reference's prefill runs its per-token kernels in a loop,
  * kernels.metal:1111-1278). Buffers as sg_gpu_run_gdn_step, with n rows:
  *   in    [n][conv_dim + value_dim + 2 n_v]  qkv | z | b | a per token;
@@ -797,8 +816,9 @@ sg_err sg_gpu_run_gdn_step(sg_gpu *g, void *in, void *w, void *state, void *out,
  *         updated in place;
  *   out   [n][value_dim].
  * p: [0]=dk [1]=dv [2]=n_v [3]=n_k [4]=ksize [5]=flags: bit 0 tiled, bit 1
- * ssm_a is -exp(A_log), bits 2-3 the first position mod 4 (the conv reads and
- * moves the tail itself, so nothing depends on it) [6]=n [7]=eps bits. */
+ * ssm_a is -exp(A_log), bits 2-3 the first position mod 4 (the ring slot that
+ * the chunk starts at under SURGE_ONESHOT=model; otherwise the conv reads and
+ * moves the tail itself and nothing depends on it) [6]=n [7]=eps bits. */
 sg_err sg_gpu_run_gdn_chunk(sg_gpu *g, void *in, void *w, void *state, void *out, const uint32_t p[8]) {
     if (!g || !in || !w || !state || !out || !p) return (sg_err){"gpu: gdn_chunk got a NULL argument"};
     const uint32_t dk = p[0], dv = p[1], nv = p[2], nk = p[3], ks = p[4], n = p[6];
@@ -815,22 +835,40 @@ sg_err sg_gpu_run_gdn_chunk(sg_gpu *g, void *in, void *w, void *state, void *out
     if (overlap(out, in) || overlap(out, w) || overlap(out, state) || overlap(state, in) || overlap(state, w))
         return (sg_err){"gpu: gdn_chunk: buffers must not overlap"};
     void *ins[3] = {in, w, state}, *outs[2] = {state, out};
-    if (sg_failed(e = push(ins, 3))) return e;
-    /* scratch: the conv output, the scan readouts and the scan workspace */
+    bool model;
+    if (sg_failed(e = oneshot_env(&model)) || sg_failed(e = push(ins, 3))) return e;
+    /* scratch: the conv output, the scan readouts and the scan workspace;
+     * before them, for the model's form, step descriptors and the 4-slot ring */
     const uint64_t cb = (uint64_t)n * cd * 4, yb = (uint64_t)n * vd * 4, wsb = (uint64_t)sgk_delta_ws_floats(nv, n) * 4;
+    const uint64_t sb = model ? ((uint64_t)n * sizeof(sgk_step) + 255) / 256 * 256 : 0, rb = model ? 4 * cd * 4 : 0;
     void *t;
-    if (sg_failed(e = scratch(g, cb + yb + wsb, &t))) return e;
+    if (sg_failed(e = scratch(g, sb + rb + cb + yb + wsb, &t))) return e;
     hipStream_t s = g->stream;
-    float *conv = t, *y = conv + (uint64_t)n * cd, *ws = y + (uint64_t)n * vd;
+    float *ring = (float *)((char *)t + sb), *conv = ring + rb / 4, *y = conv + (uint64_t)n * cd, *ws = y + (uint64_t)n * vd;
     float *dst = DEV(state), *wp = DEV(w);
+    const uint32_t pos0 = 4 + ((p[5] >> 2) & 3);    /* the ring form's first position */
+    if (model) {
+        sgk_step *st = calloc(n, sizeof *st);
+        if (!st) return (sg_err){"gpu: gdn_chunk: out of host memory"};
+        for (uint32_t z = 0; z < n; z++) st[z].pos = pos0 + z;
+        const hipError_t he = hipMemcpy(t, st, n * sizeof *st, hipMemcpyHostToDevice);
+        free(st);
+        HIPCHK(he, "gdn_chunk descriptors");
+        for (uint64_t j = 0; j < keep; j++)         /* the tail's row j: the input of position pos0 - keep + j */
+            HIPCHK(hipMemcpyAsync(ring + ((pos0 - keep + j) & 3) * cd, dst + j * cd, cd * 4, hipMemcpyDeviceToDevice, s),
+                   "conv tail in");
+    }
     sgk_gdn d = {0};
-    d.in = DEV(in); d.conv_w = wp; d.ssm_a = wp + cd * ks; d.dt_bias = d.ssm_a + nv; d.ring = dst;
+    d.in = DEV(in); d.conv_w = wp; d.ssm_a = wp + cd * ks; d.dt_bias = d.ssm_a + nv; d.ring = model ? ring : dst;
+    d.step = model ? t : NULL;
     d.S = dst + keep * cd; d.y = y; d.n_k = nk; d.n_v = nv; d.dk = dk; d.dv = dv;
     d.conv_dim = (uint32_t)cd; d.ksize = ks; d.tiled = p[5] & 1; d.neg_exp = (p[5] >> 1) & 1;
     hipError_t he = sgk_gdn_chunk(&d, conv, (uint32_t)row, n, ws, s);
     if (he == hipSuccess)
         he = sgk_rmsnorm_gated_rows(y, (const float *)DEV(in) + cd, (uint32_t)row, d.ssm_a + 2 * nv, DEV(out), dv, nv, n,
                                     fbits(p[7]), s);
+    for (uint64_t j = 0; model && he == hipSuccess && j < keep; j++)     /* the new tail: the last keep positions' inputs */
+        he = hipMemcpyAsync(dst + j * cd, ring + ((pos0 + n - keep + j) & 3) * cd, cd * 4, hipMemcpyDeviceToDevice, s);
     return finish(g, he, outs, 2);
 }
 
@@ -955,11 +993,12 @@ sg_err sg_gpu_run_attn_prefill(sg_gpu *g, void *q, void *k, void *v, void *out, 
 }
 
 /* The prefill path's attention layer core over a chunk of n tokens at
- * positions base .. base+n-1, with the kernels prefill_chunk runs
- * (sgk_attn_prep: q_norm / k_norm, partial RoPE, K and V stored f16 at each
- * token's position; sgk_attn_flash: causal attention over keys 0 .. position,
- * deep chunks split over keys and merged by the combine, sigmoid output
- * gate), on caller buffers (no reference counterpart: the reference's
+ * positions base .. base+n-1, with prefill_chunk's kernels (sgk_attn_prep:
+ * q_norm / k_norm, partial RoPE, K and V stored f16 at each token's position;
+ * sgk_attn_flash: causal attention over keys 0 .. position, deep chunks split
+ * over keys and merged by the combine, sigmoid output gate), on caller
+ * buffers: q goes to scratch where prefill prepares it in place, the RoPE
+ * rows are the chunk's own, and the cache is in the reference layout (no reference counterpart: the reference's
  * prefill runs its attention kernels per token, kernels.metal:1021-1081;
  * here they are tested whole, as one chunk):
  *   in  [n][n_heads 2 hd + 2 n_kv hd]  the input projection's rows: per
@@ -983,11 +1022,15 @@ sg_err sg_gpu_run_attn_chunk(sg_gpu *g, void *in, void *w, void *kv, void *out, 
     if (overlap(out, in) || overlap(out, w) || overlap(out, kv) || overlap(kv, in) || overlap(kv, w))
         return (sg_err){"gpu: attn_chunk: buffers must not overlap"};
     void *ins[3] = {in, w, kv}, *outs[2] = {kv, out};
-    if (sg_failed(e = push(ins, 3))) return e;
+    bool model;
+    if (sg_failed(e = oneshot_env(&model)) || sg_failed(e = push(ins, 3))) return e;
     /* scratch: step descriptors, the chunk's RoPE rows, the normed and roped q
-     * (the caller's rows stay as they are) and the key splits' partials */
-    const uint64_t steps_b = ((uint64_t)n * sizeof(sgk_step) + 255) / 256 * 256, cs_b = ((uint64_t)n * rd * 4 + 255) / 256 * 256;
-    const uint64_t q_f = (uint64_t)n * nh * hd, ah = (uint64_t)n * nh * sgk_flash_max_splits(n);
+     * (the caller's rows stay as they are) and the key splits' partials; for
+     * the model's form the RoPE rows from position 0 and a copy of the rows,
+     * whose q is prepared in place */
+    const uint32_t cs0 = model ? 0 : base;
+    const uint64_t steps_b = ((uint64_t)n * sizeof(sgk_step) + 255) / 256 * 256, cs_b = ((cap - cs0) * rd * 4 + 255) / 256 * 256;
+    const uint64_t q_f = model ? n * row : (uint64_t)n * nh * hd, ah = (uint64_t)n * nh * sgk_flash_max_splits(n);
     void *t;
     if (sg_failed(e = scratch(g, steps_b + cs_b + (q_f + ah * (2 + hd)) * 4, &t))) return e;
     hipStream_t s = g->stream;
@@ -1004,8 +1047,13 @@ sg_err sg_gpu_run_attn_chunk(sg_gpu *g, void *in, void *w, void *kv, void *out, 
     A.steps = t; A.n_heads = nh; A.n_kv = nkv; A.hd = hd; A.rope_dim = rd;
     A.q_stride = hd; A.q_tok = nh * hd; A.out_tok = nh * hd; A.max_splits = sgk_flash_max_splits(n);
     A.ntok = n; A.seq = (uint32_t)cap; A.scale = (float)(1.0 / sqrt((double)hd)); A.prefill = 1;
-    hipError_t he = sgk_rope_rows(inv, rd, base, n, cs, t, s);
-    if (he == hipSuccess) he = sgk_attn_prep(&A, wn, wn + hd, cs, base, fbits(p[7]), s);
+    hipError_t he = sgk_rope_rows(inv, rd, base, n, cs + (uint64_t)(base - cs0) * rd, t, s);
+    if (model) {
+        A.src = NULL; A.gate = work + hd; A.gate_tok = A.gate_stride = 0; A.q_tok = (uint32_t)row; A.q_stride = 2 * hd;
+        if (he == hipSuccess) he = sgk_rope_rows(inv, rd, 0, base, cs, NULL, s);
+        if (he == hipSuccess) he = hipMemcpyAsync(work, rows, n * row * 4, hipMemcpyDeviceToDevice, s);
+    }
+    if (he == hipSuccess) he = sgk_attn_prep(&A, wn, wn + hd, cs, cs0, fbits(p[7]), s);
     if (he == hipSuccess) he = sgk_attn_flash(&A, s);
     return finish(g, he, outs, 2);
 }

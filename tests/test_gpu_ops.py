@@ -469,8 +469,8 @@ GDN_CASES = [(16, 16, 128, 128, 4, True), (48, 16, 128, 128, 4, True), (6, 2, 64
 @pytest.mark.parametrize("nv,nk,dk,dv,ks,tiled", GDN_CASES,
                          ids=[f"{a}v{b}k-dk{c}-dv{d}-ks{e}-{'tiled' if f else 'grouped'}" for a, b, c, d, e, f in GDN_CASES])
 def test_gdn_decode_step_vs_oracle(gpu, nv, nk, dk, dv, ks, tiled):
-    """The decode path's fused DeltaNet step (k_gdn_step: conv ring + SiLU,
-    q/k norms and scales, beta/decay, rank-1 update and readout of S held in
+    """The decode path's fused DeltaNet step (k_gdn_step: conv + SiLU, here on
+    the caller's tail, or on the decode's ring under SURGE_ONESHOT=model; q/k norms and scales, beta/decay, rank-1 update and readout of S held in
     registers, RMSNormGated) against ref.c's gdn_layer composed from the
     oracle: the BASELINE config (16 heads, dk = dv = 128, S N(0, 0.1), conv
     width 4; conv_dim 6144 of which 2048 per q/k/v), the 27B's 48 value heads
@@ -508,8 +508,8 @@ GDN_CHUNK_CASES = [(16, 16, 128, 128, 4, True, 37, 2), (48, 16, 128, 128, 4, Tru
 def test_gdn_prefill_chunk_vs_oracle(gpu, nv, nk, dk, dv, ks, tiled, n1, n2):
     """The prefill path's DeltaNet layer core (sg_gpu_run_gdn_chunk: the
     chunk conv k_conv_chunk, with the q/k norm inside it at dk 64 and 128
-    and k_qk_norm_chunk after it at 256; the ring k_conv_ring; the scan in
-    the build's default form, k_dm_prep + k_dm_scan on the matrix cores at
+    and k_qk_norm_chunk after it at 256; the conv tail moved on behind it; the
+    scan in the build's default form, k_dm_prep + k_dm_scan on the matrix cores at
     dk 64 and 128 and the sequential k_delta_chunk at 256, with the gates
     from the b, a columns; the RMSNormGated rows) against ref.c's gdn_layer
     composed from the oracle, token by token: the BASELINE DeltaNet config
@@ -517,8 +517,9 @@ def test_gdn_prefill_chunk_vs_oracle(gpu, nv, nk, dk, dv, ks, tiled, n1, n2):
     key heads over a 130-token chunk (eight full 16-token blocks and a
     partial one), a grouped dk 64 map, conv widths 2 and 3, and dk 32 (the
     sequential scan with the separate q/k norm pass). Two chunks in a
-    row thread the conv tail and S, the second starting at another ring slot
-    (and shorter than the conv tail in one case); outputs and S within 1e-3,
+    row thread the conv tail and S, the second shorter than the conv tail in one
+    case (under SURGE_ONESHOT=model the tail goes through a position ring and
+    the second chunk starts at another slot); outputs and S within 1e-3,
     the conv tail bit-exact (it holds the inputs)."""
     rng = np.random.default_rng(nv * 11 + dk + ks + n1)
     cd, vd = 2 * nk * dk + nv * dv, nv * dv
@@ -944,8 +945,8 @@ ATTN_CHUNK_CASES = [(24, 4, 256, 64, 1000, 150), (8, 2, 256, 64, 0, 130), (12, 4
                          ids=[f"{a}q{b}kv-hd{c}-rope{d}-base{e}-n{f}" for a, b, c, d, e, f in ATTN_CHUNK_CASES])
 def test_attn_prefill_chunk_vs_oracle(gpu, nh, nkv, hd, rd, base, n):
     """The prefill path's attention layer core (sg_gpu_run_attn_chunk:
-    k_attn_prep's q_norm / k_norm, partial RoPE from the position table and
-    f16 K/V store, then the flash pass with its key split and combine and
+    k_attn_prep's q_norm / k_norm, partial RoPE from the chunk's own rows (or a
+    table from position 0 under SURGE_ONESHOT=model) and f16 K/V store, then the flash pass with its key split and combine and
     the sigmoid output gate) against ref.c's attention mixer composed from
     the oracle token by token (RMSNorm with weight, RoPE in double, K/V
     rounded to f16, decode attention over keys 0..position, gate): the 27B's
