@@ -4510,10 +4510,14 @@ struct gx_set {
 };
 // RAW: the weights are the file's 34-byte blocks; dcol is the row's first scale
 // and dm the 17 half words to the next, wrow the row's bytes. Unaligned rows
-// and a scale per line cost the product some 28 us per 512 tokens of 17408 x
-// 5120 where a repack costs 47 (the call: 247 -> 228 us), so a caller's blocks
-// are multiplied as they are up to GX_RAW_TOKENS and repacked past that.
-#define GX_RAW_TOKENS 768
+// and a scale per line cost the product with its tokens, a repack a fixed time,
+// so a caller's blocks are multiplied as they are up to GX_RAW_TOKENS (five
+// token tiles) and repacked past that. A call of 17408 x 5120 | 5120 x 17408 |
+// 12288 x 5120 | 6144 x 2048 in us, as they are: 98 | 174 | 72 | 44 at 128
+// tokens, 244 | 243 | 186 | 66 at 512, 299 | 319 | 194 | 69 at 640, 352 | 577 |
+// 256 | 94 at 768; repacked: 127 | 180 | 100 | 47, 253 | 252 | 187 | 63, 297 |
+// 314 | 202 | 68, 346 | 531 | 246 | 81.
+#define GX_RAW_TOKENS 640
 template <bool RAW>
 __device__ __forceinline__ void gx_request(gx_set &st, const v4u *xhr, size_t xb, const uint16_t *dcol, uint32_t dm,
                                            uint32_t blk, uint32_t r64) {

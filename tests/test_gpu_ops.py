@@ -739,12 +739,13 @@ def test_matmul_q8_prefill_gemm(gpu, N, M, K):
 
 
 @pytest.mark.parametrize("N,M,K", [(2, 5, 32), (16, 127, 160), (17, 129, 96), (33, 260, 1120), (48, 31, 6144),
-                                   (49, 128, 2080), (64, 385, 64), (80, 257, 544), (81, 130, 288), (769, 33, 64)])
+                                   (49, 128, 2080), (64, 385, 64), (80, 257, 544), (81, 130, 288), (769, 33, 64), (640, 33, 64),
+                                   (641, 33, 64)])
 def test_matmul_q8_few_tokens(gpu, N, M, K):
     """The few-token product at the edges of its token tiles, of its 128-row
     tiles and of its four-block stages (K / 32 from 1 to 192, split over K
     where that is at least 16 blocks each, up to 12 ways), the first count past
-    it and the first that is repacked; the split of x holds to 2^-17 a term, so 1e-4 of the largest value."""
+    it, the last that runs on blocks and the first that is repacked; the split of x holds to 2^-17 a term, so 1e-4 of the largest value."""
     rng = np.random.default_rng(N + M + K)
     X = rng.standard_normal(N * K).astype(np.float32)
     raw = q8_matrix(rng, M, K, sigma=1.0)
