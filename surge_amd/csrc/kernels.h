@@ -169,7 +169,7 @@ typedef struct {
     int per_head;
     /* The last fields are the chunk path's only, behind what the decode kernels
      * read of their arguments. Strides of the gate's rows per token and head
-     * (0: as q). */
+     * (0: as q); the combine, which reads no q, gets them in q_tok and q_stride. */
     uint32_t gate_tok, gate_stride;
     /* prep: where the projection's rows (q|gate|k|v) are read when not in place:
      * token z's at src + z*src_tok, query head h's at + h*src_stride, k and v

@@ -551,7 +551,8 @@ __global__ void __launch_bounds__(TPB) k_gemv_ring(sgk_gemv a) {
 // the block's scale. RAW_U half blocks of both rows are in flight per lane, the
 // first ones requested before x is staged. Lanes, chunks and summation order
 // are k_gemv_q8's (k_repack_q8, then the GEMV on the planes, before: 18.2 + 5.4
-// us at 4096 x 4096, now 6.7; 94 MB at 5120 columns 127 + 18, now 27). Four half
+// us at 4096 x 4096, now 6.6; 17408 x 5120 127 + 18, now 28, 3.4 TB/s: the
+// planes' aligned rows still stream faster, but not by a repack). Four half
 // blocks in flight instead of two took 80 registers and 8.3 and 33 us; x in the
 // chunked LDS layout 85 -> 89 us over 151936 x 2048.
 // ---------------------------------------------------------------------------
@@ -1262,8 +1263,10 @@ static inline sgk_attn kv_resolved(const sgk_attn *a) {
 // RoPE rows: one thread per (position, frequency). Bound by the latency of one
 // double sincos; the host loop it replaces took 0.78 us per position (32
 // frequencies, one core: 25 ms of a 26.7 ms attention chunk at 32k keys). The
-// inverse frequencies come from the host so that the angle, and with it the
-// stored float, is the same one the host's table had.
+// inverse frequencies come from the host so that the angle is the one a host
+// table would have; the stored float is its sine or cosine in double, rounded
+// (device and host libraries may differ in the double's last bit, so rarely in
+// the float's).
 struct rope_inv { double f[SGK_ROPE_HALF]; };
 __global__ void __launch_bounds__(TPB) k_rope_rows(rope_inv inv, uint32_t half, uint32_t base, uint32_t n, float *cs,
                                                    sgk_step *steps) {
@@ -2509,6 +2512,9 @@ extern "C" hipError_t sgk_attn_combine(const sgk_attn *a, hipStream_t s);
 // tiles (128 keys) each. Its partials are few then, so the combine stays short;
 // at 96 pairs (a 512-token chunk) the combine's 25 MB cost what the split saved.
 // 77 tokens of 8 heads at 1024 keys, whole layer call: 54.6 us in 3 splits, 45.5 in 8.
+// SGK_SHORT_CHUNK bounds the memory for such partials and is no turning point:
+// 8 heads over 8192 keys take 60 us at 128 tokens and 95 at 129 (67 if split
+// further), 101 at 256 (78); 24 heads fill the chip at 129 and take the same.
 #define FA_SPLIT_KEYS 512u
 static uint32_t flash_splits(const sgk_attn *a, uint32_t hw) {
     if (!a->m || !a->s || !a->acc || a->max_splits < 2) return 1;
@@ -2933,7 +2939,7 @@ __global__ void __launch_bounds__(TPB) k_gdn_finish(sgk_gdn a) {
 // multiple of that) and k_gdn_finish. Bound by latency, so by launches: the
 // ring form's one workgroup per head, with the descriptor copied in and the
 // tail copied to the ring and back around it, took 25.2 us a call at 16 heads
-// of 128 x 128 (step 7.4 us, three copies); this takes 18.4, some 10 of them
+// of 128 x 128 (step 7.4 us, three copies); this takes 18.0, some 10 of them
 // the launches and the wait.
 extern "C" hipError_t sgk_gdn_step_tail(const sgk_gdn *a, hipStream_t s) {
     if (a->ksize < 1 || a->ksize > 4 || !a->n_k || a->n_v % a->n_k) return hipErrorInvalidValue;
@@ -3086,15 +3092,15 @@ extern "C" hipError_t sgk_rmsnorm_gated(const float *y, const float *z, const fl
 // in decode). Thread (channel, block of CC_TOK tokens): the taps of token z
 // are the chunk's own inputs for positions inside the chunk, else the ring
 // slots; each output is the taps in order, then the current input (the
-// decode step's arithmetic). The ring is only read here: k_conv_ring writes
-// the chunk's last inputs into it afterwards.
+// decode step's arithmetic). The ring is only read here: conv_window moves it
+// on afterwards.
 // With hw = 1 or 2 the q and k heads (channels below qk_end, hw waves of
 // dk = 64 hw channels each, so no head crosses a workgroup) also get k_qk_norm_chunk's
 // RMS and scale before they are written: each wave sums its squares with
 // wave_sum, and a head's waves are added in block_sum's order (the same
 // per-lane values in the same lanes, so the same bits as the separate pass).
 // TAIL: the positions before the chunk are a caller's tail instead ([ksize-1]
-// [cd], oldest first; k_conv_tail moves it on afterwards).
+// [cd], oldest first; conv_window moves it on afterwards too).
 // CC tokens per thread: 16 (three inputs re-read per sixteen), or 4 while that
 // leaves most of the chip without a workgroup (a thread's loads, its 16 SiLUs
 // and a q/k wave's 16 sums are one serial chain: 45 tokens of 6144 channels 9.5 -> 5.2 us). 512 tokens of
@@ -3999,11 +4005,6 @@ extern "C" hipError_t sgk_step_advance(sgk_step *step, uint32_t *hist, hipStream
 // B[k][j] in lane j + 16*(k/8); D[i][j] in lane j + 16*(i/4), element i%4.
 // ---------------------------------------------------------------------------
 
-// X [N][ldx] f32 -> bf16 hi and lo = x - hi (both round-to-nearest-even),
-// laid out per Q8_0 block: the 64 bf16 of block b of token n, hi (32) then lo
-// (32), at xs + (b*N + n)*64, so a K step of the GEMM reads one contiguous
-// 128-byte line per token (K % 32 == 0, ldx % 4 == 0, X 16-byte aligned).
-
 // one value of X into the split: hi = bf16(v), lo = bf16(v - hi), as k_split_bf16 rounds them
 __device__ __forceinline__ void xs_put(uint16_t *xs, uint32_t N, uint32_t n, uint32_t k, float v) {
     const __bf16 hi = (__bf16)v, lo = (__bf16)(v - (float)hi);
@@ -4011,6 +4012,10 @@ __device__ __forceinline__ void xs_put(uint16_t *xs, uint32_t N, uint32_t n, uin
     o[0] = __builtin_bit_cast(uint16_t, hi);
     o[32] = __builtin_bit_cast(uint16_t, lo);
 }
+// X [N][ldx] f32 -> bf16 hi and lo = x - hi (both round-to-nearest-even),
+// laid out per Q8_0 block: the 64 bf16 of block b of token n, hi (32) then lo
+// (32), at xs + (b*N + n)*64, so a K step of the GEMM reads one contiguous
+// 128-byte line per token (K % 32 == 0, ldx % 4 == 0, X 16-byte aligned).
 __global__ void __launch_bounds__(TPB) k_split_bf16(const float *X, uint32_t ldx, uint32_t N, uint32_t K,
                                                     uint16_t *xs) {
     const uint32_t k4 = K >> 2;
@@ -4695,17 +4700,23 @@ k_gemm_q8_wide(const uint16_t *xs, const int8_t *qs, const uint16_t *d, float *Y
 // stream: a wave owns 32 weight rows and every token, its weights go from
 // memory through the wave's own LDS into MFMA fragments, four Q8_0 blocks at a
 // time (a row's four blocks are one 128-byte line), converted to bf16 in
-// registers, with the next four in flight while these are multiplied. X (the bf16 hi | lo split) goes through LDS,
-// staged for the four waves' 128 rows at a time. K is split over workgroups
-// until about three per CU run, the partials summed in order by the reduces
-// below. Per (block, token tile, weight tile) the arithmetic is gm_tile_step's.
-// RAW: the weights are the file's 34-byte blocks (any alignment).
-// 40 tokens of 5120 x 17408 from blocks: 40 us (repack 124 us and 113 us in
-// the 128-token tile before), 8 tokens 31 us (94 MB at 3 TB/s; the blocks'
-// alignment costs some), 76 tokens 54 us; 34816 x 5120 at 76 tokens 125 (147).
-// Past 80 tokens the LDS for X leaves one workgroup a CU, and the tile
-// of the wide form is used well. Two blocks per X stage from 49 tokens on keep
-// two workgroups a CU (76 tokens: 74 -> 54 us); below that they cost 1-3%.
+// registers, with the next four in flight while these are multiplied. X (the
+// bf16 hi | lo split) goes through LDS, staged for the four waves' 128 rows at
+// a time. K is split over workgroups, the partials summed in order by the
+// reduces below. Per (block, token tile, weight tile) the arithmetic is
+// gm_tile_step's. RAW: the weights are the file's 34-byte blocks (any
+// alignment).
+// 5120 x 17408 from blocks: 8 tokens 32 us (94 MB at 3 TB/s; the blocks'
+// alignment costs some), 40 tokens 41 (repack 124 and 113 in the 128-token
+// tile before), 76 tokens 52; 34816 x 5120 in planes 81 and 115 (147).
+// Two workgroups are resident on a CU at every tile count (waves_per_eu(2, 2)
+// allots the registers so). Two blocks per X stage from 49 tokens on keep room
+// for both in the LDS (76 tokens: 74 -> 54 us); below they cost 1-3%.
+// The line at 80 tokens is as far as the kernel is built, not where it loses:
+// with six and seven tiles built (two still fit) a call of 5120 x 17408 took 80
+// and 88 us at 96 and 112 tokens (the wide form 170 and 172), 17408 x 5120 96
+// and 104 (96 and 96), a prefill of four 27B layers 1.60 and 1.76 ms (1.97 and
+// 2.00).
 #define GF_NT_MAX 5
 #define GF_TM 128
 #define GF_S_MAX 12
@@ -5071,9 +5082,13 @@ extern "C" hipError_t sgk_gemm(const sgk_gemm_args *a, hipStream_t s) {
         const int kind = gemm_kind();
         if (a->raw && (kind != GEMM_WIDE || epi != SGK_EPI_STORE)) return hipErrorInvalidValue;
         if (a->N <= 16 * GF_NT_MAX && kind == GEMM_WIDE) {
-            // three workgroups per CU, at least 16 blocks of K each, partials that fit (the
+            // up to three workgroups per CU, at least 16 blocks of K each, partials that fit (the
             // fused reduce is built for these counts): the 5120 x 17408 product of 40 tokens
-            // took 52 us in 8 splits, 40 in 12, 46 in 16
+            // took 52 us in 8 splits, 40 in 12, 46 in 16. Two are resident. Counting two (at 3 and
+            // 5 token tiles) avoids a part-filled second round for some shapes (a call of 17408 x
+            // 5120 at 40 and 76 tokens 69 -> 63 and 86 -> 77 us) but leaves the 27B's 272 gate|up
+            // tiles in one split on half the places: a prefill of four of its layers 1136 -> 1178
+            // and 1442 -> 1468 us
             const uint32_t mt = (a->M + GF_TM - 1) / GF_TM, nbl = a->K / 32, per = max(1u, 3 * (uint32_t)device_cus() / mt);
             uint32_t S = 1;
             for (uint32_t v : {2u, 3u, 4u, 6u, 8u, (uint32_t)GF_S_MAX})
