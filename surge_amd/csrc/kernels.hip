@@ -551,7 +551,7 @@ __global__ void __launch_bounds__(TPB) k_gemv_ring(sgk_gemv a) {
 // the block's scale. RAW_U half blocks of both rows are in flight per lane, the
 // first ones requested before x is staged. Lanes, chunks and summation order
 // are k_gemv_q8's (k_repack_q8, then the GEMV on the planes, before: 18.2 + 5.4
-// us at 4096 x 4096, now 6.6; 17408 x 5120 127 + 18, now 28, 3.4 TB/s: the
+// us at 4096 x 4096, now 6.6; 17408 x 5120 127 + 18, now 29, 3.2 TB/s: the
 // planes' aligned rows still stream faster, but not by a repack). Four half
 // blocks in flight instead of two took 80 registers and 8.3 and 33 us; x in the
 // chunked LDS layout 85 -> 89 us over 151936 x 2048.
@@ -4706,9 +4706,9 @@ k_gemm_q8_wide(const uint16_t *xs, const int8_t *qs, const uint16_t *d, float *Y
 // reduces below. Per (block, token tile, weight tile) the arithmetic is
 // gm_tile_step's. RAW: the weights are the file's 34-byte blocks (any
 // alignment).
-// 5120 x 17408 from blocks: 8 tokens 32 us (94 MB at 3 TB/s; the blocks'
+// 5120 x 17408 from blocks: 8 tokens 33 us (94 MB at 2.9 TB/s; the blocks'
 // alignment costs some), 40 tokens 41 (repack 124 and 113 in the 128-token
-// tile before), 76 tokens 52; 34816 x 5120 in planes 81 and 115 (147).
+// tile before), 76 tokens 53; 34816 x 5120 in planes 80 and 114 (147).
 // Two workgroups are resident on a CU at every tile count (waves_per_eu(2, 2)
 // allots the registers so). Two blocks per X stage from 49 tokens on keep room
 // for both in the LDS (76 tokens: 74 -> 54 us); below they cost 1-3%.
